@@ -123,12 +123,12 @@ template <typename V>
 __device__ __forceinline__ bool is_sentinel(V v) {
   return to_bits<V>(v) == Sentinel<V>::bits;
 }
+// publishes v, which must not be the sentinel
 template <typename V>
-__device__ __forceinline__ void publish(V *p, V v) {
+__device__ __forceinline__ void store_ready(V *p, V v) {
   using U = typename Sentinel<V>::U;
-  U u = to_bits<V>(v);
-  if (u == Sentinel<V>::bits) u = Sentinel<V>::qnan;
-  __hip_atomic_store(reinterpret_cast<U *>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(reinterpret_cast<U *>(p), to_bits<V>(v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace dev

@@ -118,17 +118,26 @@ struct TrsvPlan {
   // tiled sync-free schedule (built when the pattern is recognised as a
   // grid): one workgroup per tile, its rows' dependencies inside the tile
   // kept in LDS. Rows are stored group by group, 64 slots per group (one
-  // per lane; slots past the group's rows are padding): the row id (-1 for
-  // padding), t_maxe 16-bit LDS indices of the values each row reads, and
-  // per precision its values and reciprocal diagonal (refreshed with the
+  // per lane; slots past the group's rows are padding): t_maxe byte
+  // addresses of the LDS values each row reads, and per precision one packed
+  // record per group (values, addresses, 1/d; refreshed with the
   // level-ordered values)
   bool tiled = false;
   int t_nparts = 0, t_ngroups = 0, t_mmax = 0, t_hmax = 0, t_maxe = 0, t_tau = 0;
   int t_rlanes = 1;  // lanes per row (kTileRowLanes for rows of more than 8 entries)
+  int t_ring = 0;    // groups whose results and right-hand sides LDS holds
   double t_remote = 0;
-  DevBuf t_gptr, t_prow, t_pcode, t_rfptr, t_rfcol, t_rfslot;
+  DevBuf t_gptr, t_pcode;
+  DevBuf t_rows;   // per block of groups: (row, place in the block), by row
+  DevBuf t_reads;  // per group, t_rstride places: (hand-over slot or -1, halo slot)
+  int t_rstride = 0;
   DevBuf t_lsrc, t_dpos;  // slot entry -> level-ordered entry; slot -> level position (-1: padding)
-  MultiValues t_val, t_dinv;
+  DevBuf t_pack[3];
+  // the values tiles read from each other: t_mstride slots per group, its
+  // shared rows first (FP64 or FP32, as the solve's vectors)
+  DevBuf t_mail;
+  int t_mstride = 0;
+  int64_t t_nmail = 0;
   unsigned t_wgs = 0;   // workgroups launched
   std::string t_why;    // why the tiled schedule was not built
   // JACOBI mode (built on first use): x = D^-1 w_k with w_0 = b and

@@ -62,6 +62,9 @@ struct TileLayout {
   int maxe = 0;    // entries per lane slot (4 or kTileMaxEntries)
   int tau = 0;     // tile edge in grid steps
   double remote_frac = 0;  // entries read from another tile
+  // most rows of one group that other tiles read; those rows come first in
+  // their group
+  int shared_max = 0;
   std::vector<int> part_gptr;  // tile p: groups [part_gptr[p], part_gptr[p+1])
   std::vector<int> grp_row;    // group g: row positions [grp_row[g], grp_row[g+1])
   std::vector<int> tperm;      // row position -> row
@@ -72,8 +75,9 @@ struct TileLayout {
   // row-order triangle (-1: pad)
   std::vector<int> tcode, tsrc;
   // group g's first reads from other tiles: [rf_ptr[g], rf_ptr[g+1]) of
-  // (rf_col: the row, rf_slot: its halo slot)
-  std::vector<int> rf_ptr, rf_col, rf_slot;
+  // (rf_col: the row, rf_slot: its halo slot, rf_grp, rf_pos: the
+  // group that solves it and its place there)
+  std::vector<int> rf_ptr, rf_col, rf_slot, rf_grp, rf_pos;
 };
 // ai/aj: 0-based strict triangle in row order; level: each row's level.
 // False (with the reason) when no tiling applies.

@@ -32,6 +32,7 @@
 // computed as a product with 1/d_i stored in the plan (within an ulp of the
 // quotient; keeps a divide off the sync-free dependency chain).
 #include <algorithm>
+#include <climits>
 #include <cstdlib>
 
 #include "dev_util.hpp"
@@ -196,41 +197,64 @@ __global__ __launch_bounds__(NT) void k_trsv_syncfree(
 }
 
 // ------------------------------------------------------- tiled schedule
-// One workgroup per tile (see tiling.cpp): wavefront 0 solves the tile's
-// groups (at most 64 rows of one level each) in level order, one lane per
-// row, reading every x_j from LDS: its own results of the last kTileWindow
-// groups or the values of other tiles (the halo), through one 16-bit LDS
-// index per entry. The rows' data is stored group by group, 64 slots per
-// group, and the solving wavefront loads it straight from HBM into
-// registers: each group's indices, values and 1/d, and b (gathered by row
-// id) kTileDepth groups ahead of the group it solves, the row ids twice as
-// far ahead. A group's dependency chain is then the x reads from LDS, the
-// products, and the LDS write and HBM store of the results (padding lanes
-// store nothing). Wavefronts 1..H fetch the other tiles' values:
-// wavefront w takes the tile's groups w-1, w-1+H, ..., polls the
-// values each group reads first (agent-scope loads of x, as in the
-// level-chunk kernel) into the halo, loading the next group's list while
-// it polls, and counts its finished groups in `s_prog[w-1]`; the solver
-// checks that count before a group's x reads. Halo slots are never reused
-// within a tile, so the fetching wavefronts run ahead freely. A wavefront's
-// LDS accesses are carried out in the order it issues them, so the solving
-// wavefront needs no wait after its own writes (a compiler-only fence keeps
-// the order in the code); the fetching wavefronts wait for their LDS writes
-// before counting a group. Every wait is bounded like the level-chunk
+// One workgroup per tile (see tiling.cpp). Wavefront 0, the solver, takes
+// the tile's groups (at most 64 rows of one level each) in level order, one
+// lane per row (or RL lanes), reading every x_j from LDS: its own results,
+// kept in a ring of `ring` groups, or the values of other tiles (the halo).
+// What bounds it is the number of instructions it issues per group: it is
+// alone on its dependency chain, one wavefront issues at most about one
+// instruction per 4-5 cycles, and a scattered access costs it about 64
+// cycles of address processing. So everything but the chain is done by the
+// other wavefronts:
+//  * wavefronts 1..H, the fetchers: poll the values of other tiles that each
+//    group reads first (agent-scope loads) into the halo. Blocks of NB
+//    consecutive groups go round the fetchers; a fetcher polls a block's
+//    values together, one lane per value, and counts the groups whose values
+//    have all arrived in s_prog. Halo slots are never reused within a tile,
+//    so the fetchers run ahead freely.
+//  * the last kTileIo wavefronts: gather b (by row id) into a ring in LDS
+//    ahead of the solver, store its results to x (by row id) behind it, and
+//    touch the cache lines of the row data it will load next, so that those
+//    loads find them in the L2. A block of kTileDepth groups at a time.
+// The solver loads its row data (values, LDS addresses, 1/d: one packed
+// record per group, every load contiguous over the lanes) into registers
+// kTileDepth groups ahead, and hands the rows that other tiles read over in
+// `mail`: mstride slots per group, the group's shared rows first, so one
+// group's hand-over is one short contiguous store and its readers poll one
+// or two lines instead of a line per row. x itself is not polled by anyone.
+// A wavefront's LDS accesses are carried out in the order it issues them, so
+// the solver needs no wait after its own writes (a compiler-only fence keeps
+// the order in the code); the others wait for their LDS writes before they
+// report. Every wait on another tile is bounded like the level-chunk
 // kernel's; a timeout sets *err.
-//
-// H, the number of fetching wavefronts, trades halo throughput against the
-// solving wavefront's share of its SIMD and the memory traffic of the
-// polls: with 7 or 8 wavefronts most SIMDs hold two, and the solver may
-// share issue with a fetcher; with 4, the solver has its SIMD to itself.
-// Rows on one lane (2-D and 7-point tiles, up to 64 rows and many halo
-// values per group) take 6; rows on kTileRowLanes lanes (box tiles, 16 rows
-// per group) take 3.
+// Measured per apply of both triangles, this form against one whose solver
+// issued every access but the polls, and whose tiles polled x: 128^3 7-point
+// IC(0) FP64 425 -> 290 us, FP32 in natural order 631 -> 253 us; 100x96x90
+// FP64 494 -> 200 us; 512^2 FP64 569 -> 372 us; 128^2 225 -> 171 us; 27-point
+// ILU(1) 56^3 FP32 740 -> 447 us, 90^3 FP64 1470 -> 929 us. A group takes the
+// solver 0.12-0.13 us (0.245 us before), and a hand-over about 1 us at the
+// median; the chain of hand-overs between tiles and of groups inside them is
+// what bounds the solve now. (With the hand-over slots alone the 3-D solves
+// gained 20-40%, but 512^2 lost 8%: one more store per group on the solver.)
 constexpr int kTileLanes = 64;
-constexpr int kTileHalo = 6;      // fetching wavefronts for rows on one lane
-constexpr int kTileHaloWide = 3;  // for rows on kTileRowLanes lanes
-constexpr int kTileDepth = 8;   // groups whose rows sit in registers
-constexpr int kTileXl = kTileWindow * kTileLanes;  // result slots; kTileXl is the zero slot
+constexpr int kTileDepth = 8;  // groups whose rows sit in registers; one block of the I/O wavefronts
+constexpr int kTileIo = 2;     // I/O wavefronts
+constexpr int kTileCtl = 64;   // bytes of LDS control words, ahead of the slots
+// Groups of padding the packed rows end with (the solver runs up to
+// kTileDepth - 1 groups past a tile's last one and loads kTileDepth ahead),
+// and mail slots' spare groups per tile for the same reason.
+constexpr int kTilePad = 2 * kTileDepth;
+// The I/O wavefronts touch a block's records kTileAhead blocks ahead of the
+// solver, if the records between the two, over the tiles that are active at
+// a time (groups / levels), stay within kTileTouchBytes: with more, lines are
+// displaced before they are used and the touches only add traffic. Measured
+// per apply, with / without: 512^2 FP64 (1.8 MB) 372 / 386 us, 128^2 FP64
+// 171 / 182 us, 100x96x90 FP64 (6.5 MB) 200 / 210 us, 128^3 FP32 (7.0 MB)
+// 253 / 280 us, 128^3 FP64 (10.9 MB) 310 / 290 us, 90^3 27-point ILU(1) FP64
+// (11.3 MB) 1118 / 929 us. Three blocks ahead: 2-4% slower than four.
+constexpr int kTileAhead = 4;
+constexpr int64_t kTileTouchBytes = 8 << 20;
+constexpr int kTileNever = INT_MAX / 2;  // "all groups ready"
 
 __device__ __forceinline__ void lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "local");
@@ -242,20 +266,38 @@ __device__ __forceinline__ int lds_load(const int *p) {
 __device__ __forceinline__ void lds_store(int *p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-// N bytes from p (16-byte aligned for N >= 16, 8-byte for N == 8) into out
+
+// A group's packed record: E values, E byte addresses into LDS (32-bit) and
+// 1/d per lane. Values and addresses are cut into pieces of at most 16 bytes
+// per lane, piece by piece for all 64 lanes, so that every load covers one
+// contiguous run.
+template <int E, typename T>
+struct TileRec {
+  static constexpr int kVal = E * static_cast<int>(sizeof(T));
+  static constexpr int kValPiece = kVal < 16 ? kVal : 16;
+  static constexpr int kCode = E * 4;
+  static constexpr int kCodePiece = 16;
+  static constexpr int kCodeAt = kTileLanes * kVal;
+  static constexpr int kDinvAt = kCodeAt + kTileLanes * kCode;
+  static constexpr int kBytes = kDinvAt + kTileLanes * static_cast<int>(sizeof(T));
+  static_assert(kBytes % 128 == 0, "whole cache lines");
+};
+
 typedef unsigned int tile_u2 __attribute__((ext_vector_type(2)));
 typedef unsigned int tile_u4 __attribute__((ext_vector_type(4)));
-template <int N>
-__device__ __forceinline__ void ld_bytes(const void *p, void *out) {
-  static_assert(N == 8 || N % 16 == 0, "load size");
-  if constexpr (N == 8) {
-    *reinterpret_cast<tile_u2 *>(out) =
-        __builtin_nontemporal_load(reinterpret_cast<const tile_u2 *>(p));
-  } else {
+// `total` bytes per lane in pieces of `piece` bytes; base is the same for
+// every lane
+template <int total, int piece>
+__device__ __forceinline__ void ld_pieces(const char *base, unsigned lane, void *out) {
+  static_assert(piece == 8 || piece == 16, "piece size");
 #pragma unroll
-    for (int q = 0; q < N / 16; ++q)
-      reinterpret_cast<tile_u4 *>(out)[q] =
-          __builtin_nontemporal_load(reinterpret_cast<const tile_u4 *>(p) + q);
+  for (int q = 0; q < total / piece; ++q) {
+    if constexpr (piece == 16)
+      reinterpret_cast<tile_u4 *>(out)[q] = __builtin_nontemporal_load(
+          reinterpret_cast<const tile_u4 *>(base + q * piece * kTileLanes + lane * 16u));
+    else
+      reinterpret_cast<tile_u2 *>(out)[q] = __builtin_nontemporal_load(
+          reinterpret_cast<const tile_u2 *>(base + q * piece * kTileLanes + lane * 8u));
   }
 }
 
@@ -270,177 +312,311 @@ template <> __device__ __forceinline__ float tile_val<bf16>(bf16 v) {
 }
 __device__ __forceinline__ double tile_val(double v) { return v; }
 
-// one pipeline stage: a group's slot for this lane
+// one pipeline stage: a group's record for this lane
 template <int E, typename T>
 struct TileStage {
-  alignas(16) uint16_t code[E];
+  alignas(16) uint32_t code[E];
   alignas(16) T val[E];
   T dinv;
 };
 
-template <int E, int RL, int H, typename T, typename V, typename A, bool DIAG>
-__global__ __launch_bounds__(kTileLanes * (1 + H)) void k_trsv_tiled(
-    int nparts, const int *__restrict__ gptr, const int *__restrict__ prow,
-    const uint16_t *__restrict__ pcode, const T *__restrict__ pval, const T *__restrict__ pdinv,
-    const int *__restrict__ rfptr, const int *__restrict__ rfcol, const int *__restrict__ rfslot,
-    const V *__restrict__ b, V *x, unsigned *ctl, int *err) {
-  // pipeline depth: slots of 8 entries hold twice the registers
-  constexpr int D = E <= 4 ? kTileDepth : kTileDepth * 3 / 4;
+// the LDS word at a byte address (as kept in the packed records)
+template <typename V>
+__device__ __forceinline__ const __attribute__((address_space(3))) V *lds_at(uint32_t a) {
+  return (const __attribute__((address_space(3))) V *)a;
+}
+
+// waits until *p exceeds `have`; false after kTilePolls polls, which take at
+// least kWaitTicks. No global access on this path: the solver's loads in
+// flight are counted in issue order, and a global access here would make the
+// compiler wait for all of them; nor a clock, whose read the LDS polls would
+// wait for.
+constexpr int kTilePolls = 1 << 23;  // at least 60 cycles each
+__device__ __forceinline__ bool tile_wait(const int *p, int have) {
+  for (int polls = 0; lds_load(p) <= have; ++polls) {
+    if (polls == kTilePolls) return false;
+    __builtin_amdgcn_s_sleep(0);
+  }
+  return true;
+}
+
+template <int E, int RL, int NB, int H, typename T, typename V, typename A, bool DIAG>
+__global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
+    int nparts, const int *__restrict__ gptr, const int2 *__restrict__ rows,
+    const char *__restrict__ pack, const int2 *__restrict__ reads, int rstride,
+    const V *__restrict__ b, V *__restrict__ x, V *mail, int mstride, int ring, int hmax,
+    int touch, unsigned *ctl, int *err) {
+  constexpr int D = kTileDepth;
+  static_assert(D % (NB * H) == 0, "a group's fetcher is fixed by its place in the loop");
+  static_assert(kTileIo <= kTileWindow / D, "a block's rows are listed before its results go out");
+  using R = TileRec<E, T>;
+  // LDS, all of it dynamic so that it starts at address 0 (a record's
+  // addresses are then used as they are): control words, then 8-byte slots:
+  // results of `ring` groups, the zero slot, the halo, b of `ring` groups
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int s_prog[H];
-  __shared__ int s_part, s_late;
-  V *xs = reinterpret_cast<V *>(smem);  // window, zero slot, halo
+  int *const s_prog = reinterpret_cast<int *>(smem), *const s_b = s_prog + H;
+  int &s_part = s_b[kTileIo], &s_late = s_b[kTileIo + 1], &s_done = s_b[kTileIo + 2];
+  static_assert((H + kTileIo + 3) * 4 <= kTileCtl, "control words");
   const int wave = static_cast<int>(threadIdx.x) / kTileLanes;
   const int lane = static_cast<int>(threadIdx.x) % kTileLanes;
-  for (;;) {
+  unsigned char *const bring = smem + kTileCtl + 8 * (ring * kTileLanes + 1 + hmax);
+  auto slot = [&](int q) -> V & { return *reinterpret_cast<V *>(smem + kTileCtl + 8 * q); };
+  auto bslot = [&](int q) -> V & { return *reinterpret_cast<V *>(bring + 8 * q); };
+  // The next tile's ticket and cleared control words, between two barriers.
+  // The loop below must stay one loop of whole wavefronts: thread 0's work on
+  // both sides of the back edge with no barrier between would let the
+  // compiler send the other threads ahead to the next tile without it.
+  auto next_tile = [&] {
     if (threadIdx.x == 0) {
       s_part = static_cast<int>(atomicAdd(&ctl[0], 1u));
       s_late = 0;
-      xs[kTileXl] = V(0);
+      s_done = 0;
     }
     if (threadIdx.x < H) s_prog[threadIdx.x] = 0;
+    if (threadIdx.x < kTileIo) s_b[threadIdx.x] = 0;
     __syncthreads();
-    const int p = s_part;
-    if (p >= nparts) break;
+    return __builtin_amdgcn_readfirstlane(s_part);
+  };
+  if (threadIdx.x == 0) slot(ring * kTileLanes) = V(0);
+  for (int p = next_tile(); p < nparts; p = next_tile()) {
     const int g0 = gptr[p], ng = gptr[p + 1] - g0;
-    if (wave == 0 && ng > 0) {
-      __builtin_amdgcn_s_setprio(3);  // issue priority over the halo wavefronts
-      // group j's slot of this lane (j clamped: loads past the last group
-      // repeat it, so every iteration issues the same loads)
-      auto slot_of = [&](int j) {
-        return static_cast<int64_t>(g0 + min(j, ng - 1)) * kTileLanes + lane;
-      };
-      // row ids 2D groups ahead, the rows' data and b (gathered by row id)
-      // D groups ahead
-      int rid[2 * D];
+    const int nblk = (ng + D - 1) / D;
+    if (wave == 0) {
+      __builtin_amdgcn_s_setprio(3);  // issue priority over the other wavefronts
       TileStage<E, T> st[D];
-      V bv[D];
-      auto load_rows = [&](int k, int j, int rk) {  // rk: the ring slot of j's row id
-        const int64_t sl = slot_of(j);
-        ld_bytes<E * 2>(pcode + sl * E, st[k].code);
-        ld_bytes<E * static_cast<int>(sizeof(T))>(pval + sl * E, st[k].val);
-        if constexpr (DIAG) st[k].dinv = pdinv[sl];
-        bv[k] = b[max(rid[rk], 0)];
+      int64_t at = static_cast<int64_t>(g0) * R::kBytes;
+      auto load_rows = [&](int k) {  // the next group's record
+        // (the offset is kept in scalar registers: scalar additions instead
+        // of 64-bit vector address arithmetic per load)
+        asm volatile("" : "+s"(at));
+        const char *rec = pack + at;
+        ld_pieces<R::kVal, R::kValPiece>(rec, lane, st[k].val);
+        ld_pieces<R::kCode, R::kCodePiece>(rec + R::kCodeAt, lane, st[k].code);
+        if constexpr (DIAG)
+          st[k].dinv = *reinterpret_cast<const T *>(rec + R::kDinvAt +
+                                                    static_cast<unsigned>(lane) * sizeof(T));
+        at += R::kBytes;
       };
-      // prime in the order the loop keeps, so that the loads in flight
-      // when the loop starts are as old as in any later pass (the
-      // compiler's count of loads allowed in flight then stays high;
-      // sched_barrier keeps the scheduler from reordering them)
-#pragma unroll
-      for (int k = 0; k < 2 * D; ++k) rid[k] = __builtin_nontemporal_load(prow + slot_of(k));
-      __builtin_amdgcn_sched_barrier(0);
+      // sched_barrier keeps the scheduler from reordering the groups' loads,
+      // so that the loads in flight when the loop starts are as old as in
+      // any later pass (the compiler's count of loads allowed in flight then
+      // stays high)
 #pragma unroll
       for (int k = 0; k < D; ++k) {
-        load_rows(k, k, k);
+        load_rows(k);
         __builtin_amdgcn_sched_barrier(0);
       }
-      int rdy = lds_load(&s_prog[0]);
-      for (int i0 = 0; i0 < ng; i0 += 2 * D) {
+      // the group's hand-over slots (each tile has kTileDepth groups of spare
+      // ones, so groups past the last one need no test)
+      V *mg = mail + (static_cast<int64_t>(g0) + static_cast<int64_t>(p) * D) * mstride;
+      const bool shared = lane % RL == 0 && lane / RL < mstride;
+      // A group's LDS reads are issued right behind the previous group's
+      // write, the fetcher's count first: reads are carried out in order, so
+      // values read after a sufficient count are good, and are read again
+      // in the rare other case. Hand-over and loads are issued while those
+      // reads are on their way.
+      V bv, xv[E];
+      auto read_row = [&](const TileStage<E, T> &g, int bpos) {
+        bv = bslot(bpos);
 #pragma unroll
-        for (int k2 = 0; k2 < 2 * D; ++k2) {
-          // groups past the last one (at most 2D - 1) repeat its work
-          // without publishing: a loop without early exits keeps the
-          // compiler's count of loads in flight across iterations
-          const int i = i0 + k2, k = k2 % D;
-          const bool real = i < ng;
-          // the halo values of group i are in LDS once its fetcher has
+        for (int e = 0; e < E; ++e) xv[e] = *lds_at<V>(g.code[e]);
+      };
+      if (nblk > 0 && !tile_wait(&s_b[0], 0)) s_late = 1;
+      lds_fence();
+      int rdy = lds_load(&s_prog[0]), rdb = 0;
+      code_order();
+      read_row(st[0], lane);
+      // groups past the last one (at most D - 1) repeat whatever follows in
+      // the arrays; nothing reads their results. A loop without early exits
+      // keeps the compiler's count of loads in flight across iterations.
+      for (int blk = 0; blk < nblk; ++blk) {
+        lds_store(&s_done, blk * D);
+        const int base = (blk * D & (ring - 1)) * kTileLanes + lane;
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+          // the halo values of the group are in LDS once its fetcher has
           // counted it
-          if (real && rdy <= i / H) {
-            // no global access on this path: the loads in flight are
-            // counted in issue order, and a global access here would make
-            // the compiler wait for all of them
-            const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-            for (unsigned polls = 1; lds_load(&s_prog[i % H]) <= i / H; ++polls) {
-              __builtin_amdgcn_s_sleep(0);
-              if ((polls & 1023u) == 0 && __builtin_amdgcn_s_memrealtime() - t0 > kWaitTicks) {
-                s_late = 1;
-                break;
-              }
-            }
+          constexpr int per = D / (NB * H);  // blocks of a fetcher per pass
+          const int f = (k / NB) % H, need = (blk * per + k / (NB * H)) * NB + k % NB;
+          if (rdy <= need) {
+            if (!tile_wait(&s_prog[f], need)) s_late = 1;
             lds_fence();
+            read_row(st[k], base + k * kTileLanes);
           }
-          code_order();
-          V xv[E];
-#pragma unroll
-          for (int e = 0; e < E; ++e) xv[e] = xs[st[k].code[e]];
           A acc = A(tile_val(st[k].val[0])) * A(xv[0]);
 #pragma unroll
           for (int e = 1; e < E; ++e) acc += A(tile_val(st[k].val[e])) * A(xv[e]);
           // a row on RL lanes: every lane gets the same sum (the first
           // lane's result is the one read and published)
           acc = group_sum<RL>(acc);
-          A v = A(bv[k]) - acc;
+          A v = A(bv) - acc;
           if constexpr (DIAG) v = v * A(tile_val(st[k].dinv));
           const V out = V(v);
-          const int r = rid[k2];
-          xs[(i % kTileWindow) * kTileLanes + lane] = out;
-          if (real && r >= 0) publish(x + r, out);
+          slot(base + k * kTileLanes) = out;
           code_order();
-          rdy = lds_load(&s_prog[(i + 1) % H]);
-          // refill: the row id of group i + 2D, the rows of group i + D
-          rid[k2] = __builtin_nontemporal_load(prow + slot_of(i + 2 * D));
-          load_rows(k, i + D, (k2 + D) % (2 * D));
-        }
-      }
-    } else if (wave > 0) {
-      // this wavefront's groups j = hw, hw + H, ... (hw = wave - 1): the
-      // next group's list (its halo sources and slots) is loaded while the
-      // current group's values are polled
-      const int hw = wave - 1;
-      int j = hw, f0 = 0, f1 = 0, col = 0, slot = 0;
-      if (j < ng) {
-        f0 = rfptr[g0 + j];
-        f1 = rfptr[g0 + j + 1];
-        if (f0 + lane < f1) {
-          col = rfcol[f0 + lane];
-          slot = rfslot[f0 + lane];
-        }
-      }
-      for (; j < ng; j += H) {
-        V xv = V(0);
-        if (f0 + lane < f1) xv = load_ready(x + col);
-        const int jn = j + H;
-        int nf0 = 0, nf1 = 0, ncol = 0, nslot = 0;
-        if (jn < ng) {
-          nf0 = rfptr[g0 + jn];
-          nf1 = rfptr[g0 + jn + 1];
-          if (nf0 + lane < nf1) {
-            ncol = rfcol[nf0 + lane];
-            nslot = rfslot[nf0 + lane];
+          if (k == D - 2) rdb = lds_load(&s_b[(blk + 1) % kTileIo]);
+          if (k == D - 1 && blk + 1 < nblk && rdb <= (blk + 1) / kTileIo) {
+            if (!tile_wait(&s_b[(blk + 1) % kTileIo], (blk + 1) / kTileIo)) s_late = 1;
+            lds_fence();
           }
+          rdy = lds_load(&s_prog[((k + 1) / NB) % H]);
+          code_order();
+          read_row(st[(k + 1) % D], k + 1 < D ? base + (k + 1) * kTileLanes
+                                              : ((blk + 1) * D & (ring - 1)) * kTileLanes + lane);
+          code_order();
+          // an arithmetic result is never the sentinel: it is a signalling
+          // NaN, and arithmetic returns quiet ones (IEEE mode, the default
+          // of every kernel)
+          if (shared) store_ready(mg + lane / RL, out);
+          mg += mstride;
+          load_rows(k);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        for (int t = f0 + lane; t < f1; t += kTileLanes) {
-          const int c = t == f0 + lane ? col : rfcol[t];
-          if (t != f0 + lane) xv = load_ready(x + c);
-          if (is_sentinel(xv)) {
-            const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-            for (unsigned polls = 1; is_sentinel(xv); ++polls) {
-              __builtin_amdgcn_s_sleep(1);
-              xv = load_ready(x + c);
-              if ((polls & 255u) == 0 &&
-                  (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
-                   __builtin_amdgcn_s_memrealtime() - t0 > kWaitTicks)) {
-                __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                xv = V(0);
-                break;
+      }
+      lds_store(&s_done, kTileNever);
+    } else if (wave <= H) {
+      // blocks hw, hw + H, ... of NB groups. A group's list has rstride places
+      // (x: its hand-over slot, -1 past the list; y: its halo slot), so a
+      // block's places are one run whose address needs no look-up; the lists
+      // of the next two blocks are on their way while one is polled
+      const int hw = wave - 1, nfb = (ng + NB - 1) / NB, places = NB * rstride;
+      const int lane_grp = lane / rstride;
+      auto list = [&](int jb, int q) {
+        int2 e = make_int2(-1, 0);
+        if (jb < nfb && q < places)
+          e = reads[(static_cast<int64_t>(g0) + jb * NB) * rstride + q];
+        return e;
+      };
+      int2 next = list(hw, lane), next2 = list(hw + H, lane);
+      for (int jb = hw; jb < nfb; jb += H) {
+        int2 e = next;
+        next = next2;
+        next2 = list(jb + 2 * H, lane);
+        const int done0 = jb / H * NB;
+        int grp = lane_grp, told = 0;  // the place's group; groups reported
+        for (int q = lane;; q += kTileLanes) {
+          bool pending = e.x >= 0 && jb * NB + grp < ng;
+          V xv = V(0);
+          if (pending) xv = load_ready(mail + e.x);
+          const uint64_t w0 = __builtin_amdgcn_s_memrealtime();
+          for (unsigned polls = 1;; ++polls) {
+            if (pending && !is_sentinel(xv)) {
+              slot(e.y) = xv;
+              pending = false;
+            }
+            const uint64_t left = __ballot(pending);
+            if (!left) break;
+            if constexpr (NB > 1) {
+              const int ready = __builtin_amdgcn_readlane(grp, __builtin_ctzll(left));
+              if (ready > told) {
+                told = ready;
+                lds_fence();
+                if (lane == 0) lds_store(&s_prog[hw], done0 + told);
               }
             }
+            __builtin_amdgcn_s_sleep(1);
+            if ((polls & 255u) == 0 &&
+                (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
+                 __builtin_amdgcn_s_memrealtime() - w0 > kWaitTicks)) {
+              __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              if (pending) slot(e.y) = V(0);
+              break;
+            }
+            if (pending) xv = load_ready(mail + e.x);
           }
-          xs[t == f0 + lane ? slot : rfslot[t]] = xv;
+          if (q - lane + kTileLanes >= places) break;
+          // (rare: more places than lanes)
+          e = list(jb, q + kTileLanes);
+          grp = (q + kTileLanes) / rstride;
         }
         lds_fence();
         __builtin_amdgcn_wave_barrier();
-        if (lane == 0) lds_store(&s_prog[hw], j / H + 1);
-        f0 = nf0;
-        f1 = nf1;
-        col = ncol;
-        slot = nslot;
+        if (lane == 0) lds_store(&s_prog[hw], done0 + NB);
+      }
+      lds_fence();
+      if (lane == 0) lds_store(&s_prog[hw], kTileNever);
+    } else {
+      // blocks io, io + kTileIo, ... of D groups. b of a block goes into the
+      // ring once the results of the block that held its place `ring` groups
+      // earlier are in x; the gather of the next block of this wavefront is
+      // issued before that wait. The solver's progress ends every wait here.
+      // A block's rows are listed by row id (x: the row, -1 past the last; y:
+      // its place in the block), so that neighbouring rows of b and x, which
+      // sit in different groups of the block, are accessed together: in a
+      // natural-order grid 8 runs of 8 rows per access instead of 64 single
+      // rows. Every line of such an access costs the CU's address unit a
+      // cycle or more that the polls and the solver's loads wait for.
+      const int io = wave - 1 - H, back = ring / D;
+      constexpr int NI = D / RL;  // accesses per block
+      constexpr int kTouch = (D * R::kBytes / 128 + kTileLanes - 1) / kTileLanes;
+      const int2 *const rp = rows + (static_cast<int64_t>(g0 / D) + p) * (NI * kTileLanes) + lane;
+      int2 rid[NI], rx[NI], rb[NI];
+      int tv[kTouch] = {}, tl = 0;
+      V bn[NI];
+      auto list = [&](int2(&to)[NI], int m) {
+#pragma unroll
+        for (int u = 0; u < NI; ++u) to[u] = rp[(m * NI + u) * kTileLanes];
+      };
+      auto gather = [&] {
+#pragma unroll
+        for (int u = 0; u < NI; ++u) {
+          rb[u] = rid[u];
+          bn[u] = b[max(rid[u].x, 0)];
+        }
+      };
+#pragma unroll
+      for (int u = 0; u < NI; ++u) {
+        rid[u] = rx[u] = rb[u] = make_int2(-1, 0);
+        bn[u] = V(0);
+      }
+      if (io < nblk) {
+        list(rid, io);
+        gather();
+      }
+      if (io + kTileIo < nblk) list(rid, io + kTileIo);
+      for (int m = io; m < nblk + back; m += kTileIo) {
+        const int mx = m - back;  // the block whose results go out
+        if (mx >= 0) {
+          while (lds_load(&s_done) < mx * D + D) __builtin_amdgcn_s_sleep(1);
+          lds_fence();
+          const int xb = (mx * D & (ring - 1)) * kTileLanes;
+#pragma unroll
+          for (int u = 0; u < NI; ++u)
+            if (rx[u].x >= 0) x[rx[u].x] = slot(xb + rx[u].y);
+        }
+        if (m < nblk) {
+          const int bb = (m * D & (ring - 1)) * kTileLanes;
+#pragma unroll
+          for (int u = 0; u < NI; ++u)
+            if (rb[u].x >= 0) bslot(bb + rb[u].y) = bn[u];
+          lds_fence();
+          __builtin_amdgcn_wave_barrier();
+          if (lane == 0) lds_store(&s_b[io], m / kTileIo + 1);
+        }
+        const int mt = m - back + 1 + kTileAhead;  // the block touched
+        if (touch && mt >= 0 && mt < nblk) {
+          // one lane per 128-byte line of the block's records and lists
+          const char *rec = pack + (static_cast<int64_t>(g0) + mt * D) * R::kBytes;
+#pragma unroll
+          for (int l = 0; l < kTouch; ++l) {
+            asm volatile("" ::"v"(tv[l]));
+            const int line = l * kTileLanes + lane;
+            if (line < D * R::kBytes / 128) tv[l] = *reinterpret_cast<const int *>(rec + line * 128);
+          }
+          asm volatile("" ::"v"(tl));
+          if (lane * 16 < D * rstride)
+            tl = reads[(static_cast<int64_t>(g0) + mt * D) * rstride + lane * 16].x;
+        }
+        if (m + kTileIo < nblk) gather();
+        if (m + 2 * kTileIo < nblk) list(rid, m + 2 * kTileIo);
+        const int nx = m + kTileIo - back;
+        if (nx >= 0 && nx < nblk) list(rx, nx);
       }
     }
-    __syncthreads();
-    // a solver wait that ran out of time is reported here
-    if (threadIdx.x == 0 && s_late)
+    // a wait of the solver that ran out of time
+    if (wave == 0 && s_late && lane == 0)
       __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
   }
 }
 
@@ -488,26 +664,73 @@ void sf_launch(TrsvPlan &P, const T *val, const T *diag, const V *b, V *x, hipSt
                      P.nchunks, P.chunk_start.as<int>(), rp, cl, val, diag, pm, b, x, ctl, err);
 }
 
-// x <- sentinel, control words reset (the tiled schedule's stand-in for
-// k_fill_sentinel)
+// the hand-over slots <- sentinel, control words reset
 template <typename V>
-__global__ void k_tile_prep(int64_t n, V *x, unsigned *ctl) {
+__global__ void k_tile_prep(int64_t n, V *mail, unsigned *ctl) {
   using U = typename Sentinel<V>::U;
-  U *xb = reinterpret_cast<U *>(x);
+  U *m = reinterpret_cast<U *>(mail);
   for (int64_t t = static_cast<int64_t>(blockIdx.x) * kB + threadIdx.x; t < n;
        t += static_cast<int64_t>(gridDim.x) * kB)
-    xb[t] = Sentinel<V>::bits;
+    m[t] = Sentinel<V>::bits;
   if (blockIdx.x == 0 && threadIdx.x < 16) ctl[threadIdx.x] = 0;
 }
 
-inline size_t tile_lds_bytes(int h_max, size_t vsize) {
-  return (static_cast<size_t>(kTileXl) + 1 + h_max) * vsize;
+// 8-byte LDS slots: results and b of `ring` groups, the zero slot, the halo
+inline size_t tile_lds_bytes(int ring, int h_max) {
+  return kTileCtl + 8 * (2 * static_cast<size_t>(ring) * kTileLanes + 1 + h_max);
 }
 
-template <int E, int RL, int H, typename T, typename V, typename A, bool DIAG>
+// The packed records: slot t's entries from the level-ordered values
+// (src, -1: padding), LDS addresses and reciprocal diagonal (dpos).
+template <int E, typename T>
+__global__ void k_tile_pack(int64_t slots, const int *__restrict__ src,
+                            const int *__restrict__ code, const int *__restrict__ dpos,
+                            const T *__restrict__ val, const T *__restrict__ dinv, char *out) {
+  using R = TileRec<E, T>;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t >= slots) return;
+  const int lane = static_cast<int>(t % kTileLanes);
+  char *rec = out + t / kTileLanes * R::kBytes;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int q = src[t * E + e];
+    constexpr int sT = static_cast<int>(sizeof(T));
+    const int vb = e * sT, cb = e * 4;
+    *reinterpret_cast<T *>(rec + vb / R::kValPiece * R::kValPiece * kTileLanes +
+                           lane * R::kValPiece + vb % R::kValPiece) = q >= 0 ? val[q] : T();
+    *reinterpret_cast<int *>(rec + R::kCodeAt + cb / R::kCodePiece * R::kCodePiece * kTileLanes +
+                             lane * R::kCodePiece + cb % R::kCodePiece) = code[t * E + e];
+  }
+  T d = T();
+  if (dinv && dpos[t] >= 0) d = dinv[dpos[t]];
+  *reinterpret_cast<T *>(rec + R::kDinvAt + lane * sizeof(T)) = d;
+}
+
+template <int E, typename T>
+void tile_pack(TrsvPlan &P, hipStream_t s) {
+  constexpr la_dtype dt = TileDt<T>::v;
+  const int64_t groups = P.t_ngroups + kTilePad, slots = groups * kTileLanes;
+  if (!P.t_pack[dt].p)
+    P.t_pack[dt].alloc(static_cast<size_t>(groups) * TileRec<E, T>::kBytes);
+  hipLaunchKernelGGL((k_tile_pack<E, T>), dim3(static_cast<unsigned>((slots + kB - 1) / kB)),
+                     dim3(kB), 0, s, slots, P.t_lsrc.as<int>(), P.t_pcode.as<int>(),
+                     P.t_dpos.as<int>(), P.val.v[dt].as<T>(),
+                     P.unit ? nullptr : P.diag.v[dt].as<T>(), P.t_pack[dt].as<char>());
+  LA_HIP(hipGetLastError());
+}
+
+// the packed records of one precision follow the level-ordered values
+void tile_pack(TrsvPlan &P, la_dtype dt, hipStream_t s) {
+  const bool e4 = P.t_maxe == 4;
+  if (dt == LA_F64) e4 ? tile_pack<4, double>(P, s) : tile_pack<kTileMaxEntries, double>(P, s);
+  else if (dt == LA_F32) e4 ? tile_pack<4, float>(P, s) : tile_pack<kTileMaxEntries, float>(P, s);
+  else e4 ? tile_pack<4, bf16>(P, s) : tile_pack<kTileMaxEntries, bf16>(P, s);
+}
+
+template <int E, int RL, int NB, int H, typename T, typename V, typename A, bool DIAG>
 void tiled_launch(TrsvPlan &P, const V *b, V *x, hipStream_t s) {
-  auto kern = k_trsv_tiled<E, RL, H, T, V, A, DIAG>;
-  const size_t lds = tile_lds_bytes(P.t_hmax, sizeof(V));
+  auto kern = k_trsv_tiled<E, RL, NB, H, T, V, A, DIAG>;
+  const size_t lds = tile_lds_bytes(P.t_ring, P.t_hmax);
   static size_t lds_set = 0;  // per instantiation: the largest size allowed so far
   if (lds > lds_set) {
     LA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
@@ -515,15 +738,16 @@ void tiled_launch(TrsvPlan &P, const V *b, V *x, hipStream_t s) {
                                static_cast<int>(lds)));
     lds_set = lds;
   }
-  const T *tv = static_cast<const T *>(P.t_val.get(TileDt<T>::v));
-  const T *td = DIAG ? static_cast<const T *>(P.t_dinv.get(TileDt<T>::v)) : nullptr;
-  const unsigned fg = static_cast<unsigned>(std::min<int64_t>(4096, (P.n + kB - 1) / kB));
-  hipLaunchKernelGGL(k_tile_prep<V>, dim3(std::max(fg, 1u)), dim3(kB), 0, s,
-                     static_cast<int64_t>(P.n), x, P.counter.as<unsigned>());
-  hipLaunchKernelGGL(kern, dim3(P.t_wgs), dim3(kTileLanes * (1 + H)), lds, s,
-                     P.t_nparts, P.t_gptr.as<int>(), P.t_prow.as<int>(),
-                     P.t_pcode.as<uint16_t>(), tv, td, P.t_rfptr.as<int>(), P.t_rfcol.as<int>(),
-                     P.t_rfslot.as<int>(), b, x, P.counter.as<unsigned>(), P.err_flag.as<int>());
+  const int64_t active = P.t_ngroups / std::max(P.nlevels, 1) + 1;
+  const int touch = active * P.t_ring * TileRec<E, T>::kBytes <= kTileTouchBytes ? 1 : 0;
+  const unsigned fg = static_cast<unsigned>(std::min<int64_t>(1024, (P.t_nmail + kB - 1) / kB));
+  hipLaunchKernelGGL(k_tile_prep<V>, dim3(std::max(fg, 1u)), dim3(kB), 0, s, P.t_nmail,
+                     P.t_mail.as<V>(), P.counter.as<unsigned>());
+  hipLaunchKernelGGL(kern, dim3(P.t_wgs), dim3(kTileLanes * (1 + H + kTileIo)), lds, s,
+                     P.t_nparts, P.t_gptr.as<int>(), P.t_rows.as<int2>(),
+                     P.t_pack[TileDt<T>::v].template as<const char>(), P.t_reads.as<int2>(),
+                     P.t_rstride, b, x, P.t_mail.as<V>(), P.t_mstride, P.t_ring, P.t_hmax, touch,
+                     P.counter.as<unsigned>(), P.err_flag.as<int>());
 }
 
 template <typename T, typename V, typename A, bool DIAG>
@@ -531,9 +755,13 @@ void launch_syncfree(TrsvPlan &P, const T *val, const T *diag, const V *b, V *x,
   const int64_t n = P.n;
   if (P.tiled) {
     constexpr int E8 = kTileMaxEntries, RW = kTileRowLanes;
-    if (P.t_maxe == 4) tiled_launch<4, 1, kTileHalo, T, V, A, DIAG>(P, b, x, s);
-    else if (P.t_rlanes == 1) tiled_launch<E8, 1, kTileHalo, T, V, A, DIAG>(P, b, x, s);
-    else tiled_launch<E8, RW, kTileHaloWide, T, V, A, DIAG>(P, b, x, s);
+    // fetchers: two with blocks of four groups, or four with blocks of two
+    // where a group takes longer (up to 18 values each). Measured per apply,
+    // 4 x 1 / 4 x 2 / 2 x 4 (fetchers x groups): 512^2 428 / 400 / 393 us,
+    // 56^3 27-point FP32 525 / 472 / 582 us
+    if (P.t_maxe == 4) tiled_launch<4, 1, 4, 2, T, V, A, DIAG>(P, b, x, s);
+    else if (P.t_rlanes == 1) tiled_launch<E8, 1, 4, 2, T, V, A, DIAG>(P, b, x, s);
+    else tiled_launch<E8, RW, 2, 4, T, V, A, DIAG>(P, b, x, s);
     LA_HIP(hipGetLastError());
     return;
   }
@@ -729,33 +957,10 @@ void jacobi_solve(TrsvPlan &T, la_dtype val, la_dtype vec, const void *b, void *
   jac_scale(n, val, vec, d, tmp, x, s);
 }
 
-// slot order <- level order: the plan's values (entry source index, -1 for
-// padding) and reciprocal diagonal
-__global__ void k_tile_gather(int64_t m, const int *__restrict__ src, const double *__restrict__ f,
-                              double *out) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t < m) out[t] = src[t] >= 0 ? f[src[t]] : 0.0;
-}
-
 void tiled_refresh(TrsvPlan &T, hipStream_t s) {
   if (!T.tiled) return;
-  const int64_t slots = static_cast<int64_t>(T.t_ngroups) * kTileLanes;
-  const int64_t m = slots * T.t_maxe;
-  if (T.nnz) {
-    double *tv = T.t_val.v[LA_F64].as<double>();
-    hipLaunchKernelGGL(k_tile_gather, dim3(static_cast<unsigned>((m + 255) / 256)), dim3(256), 0,
-                       s, m, T.t_lsrc.as<int>(), T.val.v[LA_F64].as<double>(), tv);
-    LA_HIP(hipGetLastError());
-    T.t_val.set_from_device_f64(tv, m, s);
-  }
-  if (!T.unit) {
-    double *td = T.t_dinv.v[LA_F64].as<double>();
-    hipLaunchKernelGGL(k_tile_gather, dim3(static_cast<unsigned>((slots + 255) / 256)),
-                       dim3(256), 0, s, slots, T.t_dpos.as<int>(),
-                       T.diag.v[LA_F64].as<double>(), td);
-    LA_HIP(hipGetLastError());
-    T.t_dinv.set_from_device_f64(td, slots, s);
-  }
+  for (int dt = 0; dt < 3; ++dt)
+    if (T.t_pack[dt].p) tile_pack(T, static_cast<la_dtype>(dt), s);
 }
 
 // The tiled schedule when the triangle's pattern is recognised as a grid
@@ -778,10 +983,12 @@ void build_tiled(TrsvPlan &P, const std::vector<int> &iperm, const std::vector<i
   LA_HIP(hipGetDevice(&dev));
   LA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   LA_HIP(hipDeviceGetAttribute(&budget, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-  // halo slots: what LDS holds beyond the window, and what a 16-bit index
-  // reaches
-  const int64_t avail = static_cast<int64_t>(budget) - static_cast<int64_t>(tile_lds_bytes(0, 8));
-  const int max_halo = static_cast<int>(std::min<int64_t>(avail / 8, 65535 - kTileXl - 1));
+  // halo slots: what LDS holds beyond the rings of kTileWindow groups (they
+  // are twice as long where the halo leaves room: the I/O wavefronts then
+  // run further ahead)
+  const int64_t avail =
+      static_cast<int64_t>(budget) - static_cast<int64_t>(tile_lds_bytes(kTileWindow, 0));
+  const int max_halo = static_cast<int>(avail / 8);
   if (max_halo < 128 || ncu < 1) {
     P.t_why = "LDS too small for the tiled schedule";
     return;
@@ -792,11 +999,17 @@ void build_tiled(TrsvPlan &P, const std::vector<int> &iperm, const std::vector<i
     return;
   const int E = L.maxe, RL = L.rlanes;
   const int G = L.ngroups;
-  const int64_t slots = static_cast<int64_t>(G) * kTileLanes, m = slots * E;
-  std::vector<int> prow(static_cast<size_t>(slots), -1), dpos(static_cast<size_t>(slots), -1);
+  // (the solve loads groups past a tile's last one)
+  const int64_t slots = static_cast<int64_t>(G + kTilePad) * kTileLanes, m = slots * E;
+  std::vector<int> dpos(static_cast<size_t>(slots), -1);
   std::vector<int> lsrc(static_cast<size_t>(m), -1);
-  std::vector<uint16_t> pcode(static_cast<size_t>(m), static_cast<uint16_t>(kTileXl));
-  std::vector<double> tv(static_cast<size_t>(m), 0.0), td(static_cast<size_t>(slots), 0.0);
+  P.t_ring = tile_lds_bytes(2 * kTileWindow, L.h_max) <= static_cast<size_t>(budget)
+                 ? 2 * kTileWindow : kTileWindow;
+  // byte addresses into LDS: the results of group i sit in place i % t_ring
+  const int zero = P.t_ring * kTileLanes;
+  std::vector<int> pcode(static_cast<size_t>(m), kTileCtl + 8 * zero), gtile(static_cast<size_t>(G));
+  for (int p = 0; p < L.nparts; ++p)
+    for (int g = L.part_gptr[p]; g < L.part_gptr[p + 1]; ++g) gtile[g] = p;
   // a row of RL lanes: its first lane carries the row id, 1/d and the
   // level position; the others only entries (no id: they publish nothing)
   for (int g = 0; g < G; ++g)
@@ -805,35 +1018,73 @@ void build_tiled(TrsvPlan &P, const std::vector<int> &iperm, const std::vector<i
         const int64_t sl = static_cast<int64_t>(g) * kTileLanes + RL * (kk - L.grp_row[g]) + w;
         const int r = L.tperm[kk];
         if (w == 0) {
-          prow[sl] = r;
           dpos[sl] = lpos[r];
-          if (!P.unit) td[sl] = 1.0 / P.h_diag[r];
         }
         for (int e = 0; e < E; ++e) {
           const size_t te = (static_cast<size_t>(kk) * RL + w) * E + e;
           const size_t pe = static_cast<size_t>(sl) * E + e;
           const int c = L.tcode[te], q = L.tsrc[te];
-          pcode[pe] = static_cast<uint16_t>(c >= 0 ? c : kTileXl + 1 + (-c - 1));
+          if (c < 0) {
+            pcode[pe] = kTileCtl + 8 * (zero + 1 + (-c - 1));
+          } else if (q >= 0) {
+            // the layout counts places modulo kTileWindow: the group is the
+            // last one before this one at that place
+            const int gi = g - L.part_gptr[gtile[g]];
+            const int gd = gi - 1 - (gi - 1 - c / kTileLanes) % kTileWindow;
+            pcode[pe] = kTileCtl + 8 * (gd % P.t_ring * kTileLanes + c % kTileLanes);
+          }
           lsrc[pe] = q >= 0 ? lrp[lpos[r]] + (q - P.h_ai[r]) : -1;
-          tv[pe] = q >= 0 ? P.h_av[q] : 0.0;
         }
       }
-  std::vector<int> rfslot(L.rf_slot.size());
-  for (size_t t = 0; t < rfslot.size(); ++t) rfslot[t] = kTileXl + 1 + L.rf_slot[t];
+  // shared rows: a fixed run of hand-over slots per group, and kTileDepth
+  // groups of spare ones per tile
+  P.t_mstride = std::max(4, (L.shared_max + 3) / 4 * 4);
+  P.t_nmail = (static_cast<int64_t>(G) + static_cast<int64_t>(L.nparts) * kTileDepth) * P.t_mstride;
+  if (P.t_nmail > INT32_MAX) {
+    P.t_why = "too many hand-over slots";
+    return;
+  }
+  // per block of kTileDepth groups its rows by row id: (row, place in the
+  // block); block m of tile p is number first group / kTileDepth + p + m
+  const int per = kTileDepth * kTileLanes / RL;
+  std::vector<int2> rows(static_cast<size_t>(G / kTileDepth + L.nparts + 1) * per,
+                         make_int2(-1, 0));
+#pragma omp parallel for schedule(dynamic, 4)
+  for (int p = 0; p < L.nparts; ++p) {
+    const int ga = L.part_gptr[p], gb = L.part_gptr[p + 1];
+    for (int g = ga; g < gb; g += kTileDepth) {
+      int2 *out = &rows[static_cast<size_t>(ga / kTileDepth + p + (g - ga) / kTileDepth) * per];
+      int2 *end = out;
+      for (int h = g; h < std::min(gb, g + kTileDepth); ++h)
+        for (int kk = L.grp_row[h]; kk < L.grp_row[h + 1]; ++kk)
+          *end++ = make_int2(L.tperm[kk], (h - g) * kTileLanes + RL * (kk - L.grp_row[h]));
+      std::sort(out, end, [](const int2 &a, const int2 &b) { return a.x < b.x; });
+    }
+  }
+  // what each group reads from other tiles: (hand-over slot, halo slot), as
+  // many places per group as the longest list has
+  int longest = 1;
+  for (int g = 0; g < G; ++g) longest = std::max(longest, L.rf_ptr[g + 1] - L.rf_ptr[g]);
+  P.t_rstride = longest;
+  std::vector<int2> reads(static_cast<size_t>(G + kTilePad) * longest, make_int2(-1, 0));
+  for (int g = 0; g < G; ++g)
+    for (int t = L.rf_ptr[g]; t < L.rf_ptr[g + 1]; ++t) {
+      const int from = L.rf_grp[t];
+      reads[static_cast<size_t>(g) * longest + t - L.rf_ptr[g]] =
+          make_int2((from + gtile[from] * kTileDepth) * P.t_mstride + L.rf_pos[t],
+                    zero + 1 + L.rf_slot[t]);
+    }
+  P.t_mail.alloc(sizeof(double) * static_cast<size_t>(P.t_nmail));
   auto up = [&](DevBuf &d, const void *h, size_t bytes) {
     d.alloc(std::max<size_t>(bytes, 4));
     d.upload(h, bytes, s);
   };
   up(P.t_gptr, L.part_gptr.data(), sizeof(int) * L.part_gptr.size());
-  up(P.t_prow, prow.data(), sizeof(int) * prow.size());
-  up(P.t_pcode, pcode.data(), sizeof(uint16_t) * pcode.size());
-  up(P.t_rfptr, L.rf_ptr.data(), sizeof(int) * L.rf_ptr.size());
-  up(P.t_rfcol, L.rf_col.data(), sizeof(int) * L.rf_col.size());
-  up(P.t_rfslot, rfslot.data(), sizeof(int) * rfslot.size());
+  up(P.t_rows, rows.data(), sizeof(int2) * rows.size());
+  up(P.t_pcode, pcode.data(), sizeof(int) * pcode.size());
+  up(P.t_reads, reads.data(), sizeof(int2) * reads.size());
   up(P.t_lsrc, lsrc.data(), sizeof(int) * lsrc.size());
   up(P.t_dpos, dpos.data(), sizeof(int) * dpos.size());
-  P.t_val.set_from_host(tv.data(), m, s);
-  if (!P.unit) P.t_dinv.set_from_host(td.data(), slots, s);
   P.t_nparts = L.nparts;
   P.t_ngroups = G;
   P.t_mmax = L.m_max;
@@ -844,6 +1095,7 @@ void build_tiled(TrsvPlan &P, const std::vector<int> &iperm, const std::vector<i
   P.t_remote = L.remote_frac;
   P.t_wgs = static_cast<unsigned>(std::min(L.nparts, ncu));
   P.tiled = true;
+  tile_pack(P, LA_F64, s);
 }
 
 hipStream_t capture_stream() {
@@ -962,10 +1214,7 @@ void trsv_add_dtype(TrsvPlan &T, la_dtype dt) {
   if (T.nnz) T.val.add(dt, T.stream);
   else if (!T.val.has[LA_F64]) { /* empty triangle: nothing stored */ }
   if (!T.unit) T.diag.add(dt, T.stream);
-  if (T.tiled) {
-    if (T.nnz) T.t_val.add(dt, T.stream);
-    if (!T.unit) T.t_dinv.add(dt, T.stream);
-  }
+  if (T.tiled && !T.t_pack[dt].p) tile_pack(T, dt, T.stream);
   if (T.transposed) trsv_add_dtype(*T.transposed, dt);
   LA_HIP(hipStreamSynchronize(T.stream));
 }

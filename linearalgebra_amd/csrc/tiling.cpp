@@ -300,9 +300,16 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
   // rows of each tile by (level, index); tiles by their first level
   std::vector<int> order(static_cast<size_t>(n));
   for (int i = 0; i < n; ++i) order[i] = i;
+  // (rows that other tiles read come first in their level, by the reading
+  // tile: the solve hands those over as one contiguous run per group)
+  std::vector<int> reader(static_cast<size_t>(n), INT32_MAX);
+  for (int i = 0; i < n; ++i)
+    for (int q = ai[i]; q < ai[i + 1]; ++q)
+      if (part[aj[q]] != part[i]) reader[aj[q]] = std::min(reader[aj[q]], part[i]);
   std::sort(order.begin(), order.end(), [&](int a, int b) {
     if (part[a] != part[b]) return part[a] < part[b];
     if (level[a] != level[b]) return level[a] < level[b];
+    if (reader[a] != reader[b]) return reader[a] < reader[b];
     return a < b;
   });
   std::vector<int> pstart(static_cast<size_t>(nparts) + 1, 0);
@@ -366,13 +373,20 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
   const int E = out.maxe;
   const int zero_slot = kTileWindow * lanes;
   std::vector<int> slot_of(static_cast<size_t>(n)), grp_of(static_cast<size_t>(n));
+  std::vector<int> pos_of(static_cast<size_t>(n)), group_id(static_cast<size_t>(n));
   for (int pi = 0; pi < nparts; ++pi)
-    for (int g = out.part_gptr[pi]; g < out.part_gptr[pi + 1]; ++g)
+    for (int g = out.part_gptr[pi]; g < out.part_gptr[pi + 1]; ++g) {
+      int shared = 0;
       for (int kk = out.grp_row[g]; kk < out.grp_row[g + 1]; ++kk) {
-        grp_of[out.tperm[kk]] = g - out.part_gptr[pi];
-        slot_of[out.tperm[kk]] =
-            ((g - out.part_gptr[pi]) % kTileWindow) * lanes + rl * (kk - out.grp_row[g]);
+        const int r = out.tperm[kk];
+        grp_of[r] = g - out.part_gptr[pi];
+        group_id[r] = g;
+        pos_of[r] = kk - out.grp_row[g];
+        slot_of[r] = ((g - out.part_gptr[pi]) % kTileWindow) * lanes + rl * pos_of[r];
+        shared += reader[r] != INT32_MAX;
       }
+      out.shared_max = std::max(out.shared_max, shared);
+    }
   out.tcode.assign(static_cast<size_t>(n) * rl * E, zero_slot);
   out.tsrc.assign(static_cast<size_t>(n) * rl * E, -1);
   out.rf_ptr.assign(1, 0);
@@ -402,6 +416,8 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
               halo_used.push_back(c);
               out.rf_col.push_back(c);
               out.rf_slot.push_back(halo_of[c]);
+              out.rf_grp.push_back(group_id[c]);
+              out.rf_pos.push_back(pos_of[c]);
             }
             code = -(halo_of[c] + 1);
           }

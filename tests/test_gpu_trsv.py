@@ -490,3 +490,55 @@ def test_tiled_schedule_off_and_non_grid(dev, monkeypatch):
     L, D, U = orc.split_ldu(F)
     fw = la.TriangularSolve(as_lib_csr(L), None, upper=False)
     assert not fw.info()["tiled"]
+
+
+def _tiled_edge_case(name):
+    if name == "long_box":  # halo past 16375 slots: the short LDS rings
+        return la.iluk(la.gen.aniso27(2090, 6, 6), 1)
+    return la.iluk(la.gen.laplace3d(int(name), 34, 33), 0)  # tiles of n + 1 .. n + 6 groups
+
+
+@pytest.mark.parametrize("name", ["40", "41", "43", "46", "47", "long_box"])
+@pytest.mark.parametrize("vec", ["f64", "f32"])
+def test_tiled_solver_blocks_and_rings(dev, name, vec):
+    """The tiled kernel's blocks of 8 groups end at, before and after a
+    tile's last group, its rings are long and short, and a right-hand side
+    that holds the hand-over sentinel's bits (a signalling NaN) still ends:
+    the rows that depend on it are NaN, all others exact. FP64: 1e-12; FP32
+    (rows of at most 31 entries, levels up to 2150): each row adds at most
+    32 roundings of 2^-24 to what its inputs carry, and the factors'
+    off-diagonal row sums stay below 1, so 32 * 2^-24 / (1 - rowsum) bounds
+    the relative error; 1e-4 covers row sums up to 0.98."""
+    import torch
+    F = _tiled_edge_case(name)
+    L, D, U = la.split_ldu(F)
+    dt = torch.float64 if vec == "f64" else torch.float32
+    tol = 1e-12 if vec == "f64" else 1e-4
+    b = la.gen.uniform(F.n, 17)
+    for T, diag, upper in ((L, None, False), (U, D, True)):
+        S = la.TriangularSolve(T, diag, upper=upper)
+        assert S.info()["tiled"], name
+        o = orc.CSR(T.n, T.ai, T.aj, T.av)
+        ref = orc.backward_sub(o, D, b) if upper else orc.forward_sub(o, b)
+        bt = torch.tensor(b, device=dev, dtype=dt)
+        x = torch.zeros_like(bt)
+        S.solve(bt, x)
+        first = x.clone()
+        err = np.abs(x.cpu().numpy() - ref).max() / np.abs(ref).max()
+        print("case", name, vec, "upper" if upper else "lower", "err", err, flush=True)
+        assert err <= tol
+        S.solve(bt, x)
+        assert torch.equal(x, first)
+        r = F.n // 2
+        if vec == "f64":
+            bt.view(torch.int64)[r] = 0x7FF4A5A5A5A5A5A5
+        else:
+            bt.view(torch.int32)[r] = 0x7FA5A5A5
+        S.solve(bt, x)
+        nan = torch.isnan(x)
+        assert bool(nan[r])
+        assert torch.equal(x[~nan], first[~nan])
+        bad = b.copy()
+        bad[r] = np.nan
+        refn = orc.backward_sub(o, D, bad) if upper else orc.forward_sub(o, bad)
+        assert np.array_equal(nan.cpu().numpy(), np.isnan(refn))
