@@ -21,12 +21,13 @@
 // Products and differences are rounded separately (no fused multiply-add),
 // as in the reference's x86-64 build.
 //
-// Rows are processed level by level (one launch per level of the
-// factorisation's dependency DAG, which is the lower triangular solve's),
-// one 64-lane workgroup per row: the row's columns and values sit in LDS;
-// for each eliminating row k the lanes take k's entries, find their column
-// in the row by binary search and update it. A row longer than kRowCap is
-// done by one lane in global memory, in the host's loop order.
+// Rows of at most 64 entries (and eliminations): one launch, sync-free
+// (k_factor_rows). Longer rows: level by level (one launch per level of the
+// factorisation's dependency DAG, which is the lower triangular solve's), one
+// 64-lane workgroup per row with the row's columns and values in LDS; for
+// each eliminating row k the lanes take k's entries, find their column in the
+// row by binary search and update it. A row longer than kRowCap is done by
+// one lane in global memory, in the host's loop order.
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -41,6 +42,7 @@
 #pragma clang fp contract(off)
 
 namespace laamd {
+using namespace dev;
 
 struct NumericPlan {
   bool ic = false;
@@ -54,7 +56,12 @@ struct NumericPlan {
   DevBuf rows;             // rows in dependency-level order
   std::vector<int> level_ptr;
   DevBuf pptr, pk, pq;     // IC: per row j the (k, q) eliminations, host order
-  DevBuf err;              // row + 1 of a failed pivot, else 0
+  DevBuf err;              // row + 1 of a failed pivot, else 0; a wait that ran out
+  // the sync-free form: lanes per row (0: not used), chunks of rows that
+  // never span a level, per factor entry its entry of A or -1, per row the
+  // diagonal's position (ILU), the ticket counter
+  int lanes = 0, nchunks = 0;
+  DevBuf chunk_start, f2a, dpos, ticket;
   std::vector<int> h_fai, h_faj;
 };
 void NumericPlanDeleter::operator()(NumericPlan *p) const { delete p; }
@@ -238,6 +245,215 @@ __global__ __launch_bounds__(64) void k_ic_rows(int k0, const int *__restrict__ 
   for (int u = lane; u < len; u += 64) fav[ps + u] = u == 0 ? d : vals[u] / d;
 }
 
+// ---------------------------------------------------------------- sync-free
+// One launch for the whole factorisation: a wavefront takes 64 / G rows, G
+// lanes each, one entry per lane, and keeps them in registers. Everything
+// that depends on the pattern alone is done first (the row's columns, where
+// each eliminating row's entries fall in it, by binary search in LDS); then
+// the values of the eliminating rows are polled as they appear (a value that
+// is no longer the sentinel is final: agent-scope relaxed loads and stores,
+// as in the sync-free solves) and applied in the host's order. Workgroups
+// claim chunks of rows in level order, so every wait is on a row of an
+// earlier ticket or a smaller level, which a running wavefront holds.
+// What bounds it is the chain of rows: per level one store-to-poll hop and
+// the divisions of the row's last eliminations. One launch per level with a
+// row's three dependent loads per elimination in the loop, against this
+// form: 27-point ILU(1) on 48^3 (612 levels, rows of up to 61 entries)
+// 20.8 -> 2.2 ms, ILU(0) 5.45 -> 1.15 ms; 72^3 IC(0) 1.55 -> 0.48 ms; 128^2
+// IC(0) (255 levels) 1.18 -> 0.36 ms (with the refreshed solve plans).
+constexpr int kFacWaves = 4;
+constexpr int kFacMaxLanes = 64;
+// workgroups: this many levels of chunks at a time (clamped to 64 .. 1024),
+// so that the pattern work of later rows is done while they wait. 27-point
+// ILU(1) on 48^3 with 1 / 2 / 4 / 8 / 16 levels ahead (8 wavefronts): 8.3 /
+// 6.1 / 3.4 / 2.3 / 2.2 ms; 72^3 IC(0) with 4 / 8 / 32: 490 / 465 / 573 us
+// (more pollers)
+constexpr int kFacAhead = 12;
+constexpr uint64_t kFacWaitTicks = 20000000;  // 0.2 s of the 100 MHz clock
+
+template <int G>
+__device__ __forceinline__ int row_bcast(int v, int l) {
+  if constexpr (G == 64) return __builtin_amdgcn_readlane(v, l);
+  else return __shfl(v, l, G);
+}
+template <int G>
+__device__ __forceinline__ double row_bcast(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const int lo = row_bcast<G>(static_cast<int>(b), l);
+  const int hi = row_bcast<G>(static_cast<int>(b >> 32), l);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
+}
+
+// src: ILU the diagonals' positions, IC the rows' elimination lists (pptr,
+// with pk and pq)
+template <int G, bool IC>
+__global__ __launch_bounds__(64 * kFacWaves) void k_factor_rows(
+    int nchunks, const int *__restrict__ chunk_start, const int *__restrict__ rows,
+    const int *__restrict__ fai, const int *__restrict__ faj, const int *__restrict__ src,
+    const int *__restrict__ pk, const int *__restrict__ pq, const int *__restrict__ f2a,
+    const double *__restrict__ av, double *fav, double diag_mul, double diag_add, int strict,
+    unsigned *ticket, int *err) {
+  constexpr int B = G < 8 ? G : 8;  // eliminations whose loads are in flight together
+  __shared__ int s_cols[kFacWaves][64];
+  __shared__ uint8_t s_map[kFacWaves][G * 64];
+  __shared__ int s_c[2];
+  const int wave = static_cast<int>(threadIdx.x) >> 6, lane = threadIdx.x & 63;
+  const int sub = lane & (G - 1), row0 = lane - sub;  // lane in the row, the row's first lane
+  int *const cols = s_cols[wave];
+  uint8_t *const map = s_map[wave];
+  if (threadIdx.x == 0) s_c[0] = static_cast<int>(atomicAdd(ticket, 1u));
+  __syncthreads();
+  for (int it = 0;; ++it) {
+    const int c = __builtin_amdgcn_readfirstlane(s_c[it & 1]);
+    if (c >= nchunks) break;
+    if (threadIdx.x == 0) s_c[(it + 1) & 1] = static_cast<int>(atomicAdd(ticket, 1u));
+    const int k = chunk_start[c] + (wave * 64 + lane) / G;
+    const bool on = k < chunk_start[c + 1];
+    if (__ballot(on)) {
+      const int i = on ? rows[k] : 0;
+      const int fb = on ? fai[i] : 0, len = on ? fai[i + 1] - fb : 0;
+      const bool mine = sub < len;
+      const int col = mine ? faj[fb + sub] : INT_MAX;
+      const int a = mine ? f2a[fb + sub] : -1;
+      double val = a >= 0 ? av[a] : 0.0;
+      cols[lane] = col;
+      // eliminations e: entries start .. start + cnt of the factor, the first
+      // of them the pivot (ILU) or this row's multiplier (IC)
+      int ne, start = 0, cnt = 0;
+      if constexpr (IC) {
+        if (sub == 0) val = diag_add != 0.0 ? val + diag_add : val * diag_mul;
+        const int e0 = on ? src[i] : 0;
+        ne = on ? src[i + 1] - e0 : 0;
+        if (sub < ne) {
+          start = pq[e0 + sub];
+          cnt = fai[pk[e0 + sub] + 1] - start;
+        }
+      } else {
+        const uint64_t low = __ballot(mine && col < i);
+        ne = G == 64 ? __popcll(low)
+                     : __popcll((low >> row0) & ((1ull << (G & 63)) - 1ull));
+        if (sub < ne) {
+          start = src[col];
+          cnt = fai[col + 1] - start;
+        }
+      }
+      int nmax = ne;  // over the wavefront's rows
+      if constexpr (G < 64) {
+#pragma unroll
+        for (int d = G; d < 64; d <<= 1) nmax = max(nmax, __shfl_xor(nmax, d, 64));
+      }
+      nmax = __builtin_amdgcn_readfirstlane(nmax);
+      // where the eliminating rows' entries fall: map[e][lane] = the entry
+      // that updates this lane's, 0xFF for none
+      for (int e = 0; e < nmax; ++e) map[e * 64 + lane] = 0xFF;
+      for (int e0 = 0; e0 < nmax; e0 += B) {
+        int cc[B], pos[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+          const int es = e0 + u < nmax ? e0 + u : nmax - 1;
+          const int st = row_bcast<G>(start, es), m = row_bcast<G>(cnt, es);
+          const bool in = e0 + u < ne && sub < m && (IC || sub > 0);
+          cc[u] = in ? faj[st + sub] : -1;
+          pos[u] = row0;
+        }
+#pragma unroll
+        for (int d = G / 2; d >= 1; d >>= 1)
+#pragma unroll
+          for (int u = 0; u < B; ++u)
+            if (cols[pos[u] + d - 1] < cc[u]) pos[u] += d;
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+          if (cc[u] >= 0 && cols[pos[u]] == cc[u])
+            map[(e0 + u) * 64 + pos[u]] = static_cast<uint8_t>(sub);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "local");
+      double v[B], vn[B];
+      int at[B], an[B];  // -1: no such elimination in this lane's row
+      bool hit[B], hn[B];
+      auto fetch = [&](int e0, double(&w)[B], int(&p)[B], bool(&h)[B]) {
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+          p[u] = -1;
+          h[u] = false;
+          w[u] = 0.0;
+          if (e0 + u < nmax) {
+            const int st = row_bcast<G>(start, e0 + u);
+            const int q = map[(e0 + u) * 64 + lane];
+            h[u] = q != 0xFF && e0 + u < ne;
+            if (e0 + u < ne) {
+              p[u] = st + (h[u] ? q : 0);
+              w[u] = load_ready(fav + p[u]);
+            }
+          }
+        }
+      };
+      if (nmax > 0) fetch(0, v, at, hit);
+      for (int e0 = 0; e0 < nmax; e0 += B) {
+        fetch(e0 + B, vn, an, hn);
+        const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
+        for (unsigned polls = 1;; ++polls) {
+          bool wait = false;
+#pragma unroll
+          for (int u = 0; u < B; ++u) wait |= at[u] >= 0 && is_sentinel(v[u]);
+          if (!__ballot(wait)) break;
+          __builtin_amdgcn_s_sleep(1);
+          if ((polls & 255u) == 0 &&
+              (__hip_atomic_load(err + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
+               __builtin_amdgcn_s_memrealtime() - t0 > kFacWaitTicks)) {
+            __hip_atomic_fetch_or(err + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
+          }
+#pragma unroll
+          for (int u = 0; u < B; ++u)
+            if (at[u] >= 0 && is_sentinel(v[u])) v[u] = load_ready(fav + at[u]);
+#pragma unroll
+          for (int u = 0; u < B; ++u)
+            if (an[u] >= 0 && is_sentinel(vn[u])) vn[u] = load_ready(fav + an[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+          const int e = e0 + u;
+          if (e >= nmax) break;
+          if constexpr (IC) {
+            const double ukj = row_bcast<G>(v[u], 0);
+            if (hit[u]) val = val - ukj * v[u];
+          } else {
+            // (the lane of column k holds the pivot: nothing updates it)
+            const double l = row_bcast<G>(val, e) / row_bcast<G>(v[u], e);
+            if (hit[u]) val = val - l * v[u];
+            if (sub == e && e < ne) val = l;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+          v[u] = vn[u];
+          at[u] = an[u];
+          hit[u] = hn[u];
+        }
+      }
+      if constexpr (IC) {
+        const double piv = row_bcast<G>(val, 0);
+        if (sub == 0 && on && (strict ? piv <= 0 : piv < 0)) flag_row(err, i);
+        const double d = sqrt(piv);
+        val = sub == 0 ? d : val / d;
+      }
+      if (mine) {
+        unsigned long long o = to_bits<double>(val);
+        if (o == Sentinel<double>::bits) o = Sentinel<double>::qnan;
+        store_ready(fav + fb + sub, from_bits<double>(o));
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// every factor value <- sentinel
+__global__ void k_factor_mark(int64_t m, double *v) {
+  for (int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < m;
+       t += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    v[t] = from_bits<double>(Sentinel<double>::bits);
+}
+
 template <typename T>
 void upload_vec(DevBuf &b, const std::vector<T> &v, hipStream_t s) {
   b.alloc(sizeof(T) * std::max<size_t>(v.size(), 1));
@@ -303,6 +519,33 @@ void finish_plans(Prec &P, NumericPlan &N, const std::vector<int> &Li, const std
   P.tmp[1].alloc(sizeof(float) * std::max(n, 1));
   LA_HIP(hipStreamSynchronize(s));
 }
+// The sync-free form applies when a row and its eliminations fit a wavefront:
+// the fewest lanes per row that hold both (at least 4).
+void plan_sync_free(NumericPlan &N, const std::vector<int> &fai, const std::vector<int64_t> &a2f,
+                    int max_elim, const std::vector<int> &dpos, hipStream_t s) {
+  int longest = max_elim;
+  for (int i = 0; i < N.n; ++i) longest = std::max(longest, fai[i + 1] - fai[i]);
+  if (longest > kFacMaxLanes || N.nnzA >= INT32_MAX) return;
+  N.lanes = 4;
+  while (N.lanes < longest) N.lanes *= 2;
+  std::vector<int> f2a(static_cast<size_t>(N.nnzF), -1), chunks;
+  for (size_t a = 0; a < a2f.size(); ++a)
+    if (a2f[a] >= 0) f2a[a2f[a]] = static_cast<int>(a);
+  const int per = kFacWaves * 64 / N.lanes;
+  for (size_t l = 0; l + 1 < N.level_ptr.size(); ++l)
+    for (int k = N.level_ptr[l]; k < N.level_ptr[l + 1]; k += per) {
+      chunks.push_back(k);
+    }
+  N.nchunks = static_cast<int>(chunks.size());
+  // a chunk ends where the next one starts: the last one of a level at the
+  // level's end, which is the next level's start
+  chunks.push_back(N.n);
+  upload_vec(N.chunk_start, chunks, s);
+  upload_vec(N.f2a, f2a, s);
+  upload_vec(N.dpos, dpos, s);
+  N.ticket.alloc(sizeof(unsigned) * 4);
+  LA_HIP(hipStreamSynchronize(s));
+}
 }  // namespace
 
 std::unique_ptr<Prec> make_prec_ilu_gpu(int n, int base, const int *ai, const int *aj, int level,
@@ -339,6 +582,7 @@ std::unique_ptr<Prec> make_prec_ilu_gpu(int n, int base, const int *ai, const in
   upload_vec(N.a2f, a2f, s);
   N.diag.alloc(sizeof(double) * std::max(n, 1));
   finish_plans(*P, N, Li, Lj, Ls, nullptr, Ui, Uj, Us, dpos, s);
+  plan_sync_free(N, fai, a2f, 0, std::vector<int>(dpos.begin(), dpos.end()), s);
   N.h_fai = std::move(fai);
   N.h_faj = std::move(faj);
   return P;
@@ -457,17 +701,45 @@ std::unique_ptr<Prec> make_prec_ic_gpu(int n, int base, const int *ai, const int
   upload_vec(N.pk, pk, s);
   upload_vec(N.pq, pq, s);
   finish_plans(*P, N, Li, Lj, Ls, &dsrc, Ui, Uj, Us, dsrc, s);
+  int max_elim = 0;
+  for (int j = 0; j < n; ++j) max_elim = std::max(max_elim, pptr[j + 1] - pptr[j]);
+  plan_sync_free(N, fai, a2f, max_elim, {}, s);
   N.h_fai = std::move(fai);
   N.h_faj = std::move(faj);
   return P;
 }
 
-void prec_refactor(Prec &P, const double *a_vals, hipStream_t s) {
-  if (!P.num) throw la_error(LA_ERR_STATE, "preconditioner was built from a host factor");
-  NumericPlan &N = *P.num;
-  LA_CHECK_ARG(a_vals || N.nnzA == 0, "null values");
-  if (N.n == 0) return;
-  LA_HIP(hipMemsetAsync(N.err.p, 0, sizeof(int) * 4, s));
+namespace {
+void factor_rows(NumericPlan &N, const double *a_vals, hipStream_t s) {
+  double *fav = N.fav.as<double>();
+  LA_HIP(hipMemsetAsync(N.ticket.p, 0, sizeof(unsigned) * 4, s));
+  hipLaunchKernelGGL(k_factor_mark, dim3(2048), dim3(256), 0, s, N.nnzF, fav);
+  LA_HIP(hipGetLastError());
+  const int levels = std::max<int>(1, static_cast<int>(N.level_ptr.size()) - 1);
+  const unsigned grid = static_cast<unsigned>(
+      std::min(N.nchunks, std::clamp(kFacAhead * N.nchunks / levels, 64, 1024)));
+  const bool add = N.ic && N.additive;
+#define LA_FAC(G, IC)                                                                          \
+  hipLaunchKernelGGL((k_factor_rows<G, IC>), dim3(grid), dim3(64 * kFacWaves), 0, s, N.nchunks, \
+                     N.chunk_start.as<int>(), N.rows.as<int>(), N.fai.as<int>(),                \
+                     N.faj.as<int>(), IC ? N.pptr.as<int>() : N.dpos.as<int>(), N.pk.as<int>(), \
+                     N.pq.as<int>(), N.f2a.as<int>(), a_vals, fav, 1.0 + N.omega,               \
+                     add ? N.omega : 0.0, add ? 1 : 0, N.ticket.as<unsigned>(), N.err.as<int>())
+#define LA_FACG(IC)                                                                            \
+  switch (N.lanes) {                                                                           \
+    case 4: LA_FAC(4, IC); break;                                                              \
+    case 8: LA_FAC(8, IC); break;                                                              \
+    case 16: LA_FAC(16, IC); break;                                                            \
+    case 32: LA_FAC(32, IC); break;                                                            \
+    default: LA_FAC(64, IC); break;                                                            \
+  }
+  if (N.ic) LA_FACG(true) else LA_FACG(false)
+#undef LA_FACG
+#undef LA_FAC
+  LA_HIP(hipGetLastError());
+}
+
+void factor_levels(NumericPlan &N, const double *a_vals, hipStream_t s) {
   double *fav = N.fav.as<double>();
   hipLaunchKernelGGL(k_fill_zero, dim3(2048), dim3(256), 0, s, N.nnzF, fav);
   if (N.nnzA)
@@ -494,10 +766,23 @@ void prec_refactor(Prec &P, const double *a_vals, hipStream_t s) {
                          N.diag.as<double>(), N.err.as<int>());
   }
   LA_HIP(hipGetLastError());
-  int bad = 0;
-  LA_HIP(hipMemcpyAsync(&bad, N.err.p, sizeof(int), hipMemcpyDeviceToHost, s));
+}
+}  // namespace
+
+void prec_refactor(Prec &P, const double *a_vals, hipStream_t s) {
+  if (!P.num) throw la_error(LA_ERR_STATE, "preconditioner was built from a host factor");
+  NumericPlan &N = *P.num;
+  LA_CHECK_ARG(a_vals || N.nnzA == 0, "null values");
+  if (N.n == 0) return;
+  LA_HIP(hipMemsetAsync(N.err.p, 0, sizeof(int) * 4, s));
+  if (N.lanes) factor_rows(N, a_vals, s);
+  else factor_levels(N, a_vals, s);
+  double *fav = N.fav.as<double>();
+  int bad[2] = {0, 0};
+  LA_HIP(hipMemcpyAsync(bad, N.err.p, sizeof(bad), hipMemcpyDeviceToHost, s));
   LA_HIP(hipStreamSynchronize(s));
-  if (bad)
+  if (bad[1]) throw la_error(LA_ERR_TIMEOUT, "sync-free factorisation exceeded its spin bound");
+  if (bad[0])
     throw la_error(LA_ERR_NUMERIC, !N.ic        ? "ILU factorisation met a row without a diagonal"
                                    : N.additive ? "IC factorisation hit a non-positive pivot"
                                                 : "IC factorisation hit a negative pivot");

@@ -207,3 +207,42 @@ def test_ilu_gpu_missing_diagonal_rejected(dev):
     with pytest.raises(la.LaError) as e:
         la.Preconditioner.ilu_gpu(A, 0)
     assert e.value.code == 5
+
+
+@pytest.mark.parametrize("width", [1, 2, 3, 4, 7, 8, 15, 16, 31, 32, 63, 64])
+@pytest.mark.parametrize("kind", ["ilu", "ic", "ick"])
+def test_banded_factor_bitwise_host(dev, width, kind):
+    """Rows of every lane count of the sync-free factorisation and one past
+    its longest (banded matrices: IC rows hold width + 1 entries and as many
+    as width eliminations, ILU rows 2 width + 1; every row depends on the
+    one before it), bitwise the host's."""
+    import torch
+    rng = np.random.default_rng(width)
+    n = 260
+    rows, cols = np.nonzero(np.abs(np.subtract.outer(np.arange(n), np.arange(n))) <= width)
+    v = rng.uniform(-1, 0, len(rows))
+    lo, hi = np.minimum(rows, cols), np.maximum(rows, cols)
+    sym = rng.uniform(-1, 0, (n, n))[lo, hi]
+    av = np.where(rows == cols, 2.0 * width + 1.5, v if kind == "ilu" else sym)
+    ai = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))])
+    A = la.CSR(n, ai, cols, av)
+    if kind == "ilu":
+        F, P = la.iluk(A, 0), la.Preconditioner.ilu_gpu(A, 0)
+    elif kind == "ic":
+        (F, ok), P = la.icc(la.split_triangle(A, True), 0), la.Preconditioner.ic_gpu(A, 0)
+    else:
+        U = la.split_triangle(A, True)
+        ia, ja = la.icc_symbolic(U, U.ai[:-1], 0)
+        (F, ok), P = la.ick_numeric(U, U.ai[:-1], ia, ja, 0.125), la.Preconditioner.ick_gpu(A, 0, 0.125)
+    for _ in range(3):
+        P.refactor(torch.tensor(A.av, device=dev))
+        G = P.factor()
+        assert np.array_equal(G.ai, F.ai) and np.array_equal(G.aj, F.aj)
+        assert np.array_equal(G.av, F.av), "max diff %.3e" % np.max(np.abs(G.av - F.av))
+    if kind != "ilu":  # a bad pivot is reported, and a good refactorisation follows
+        bad = A.av.copy()
+        bad[(rows == cols) & (rows == n // 2)] = -1.0
+        with pytest.raises(la.LaError):
+            P.refactor(torch.tensor(bad, device=dev))
+        P.refactor(torch.tensor(A.av, device=dev))
+        assert np.array_equal(P.factor().av, F.av)
