@@ -150,8 +150,18 @@ double correlation(const std::vector<int> &a, const std::vector<int> &b) {
 
 // Tiles from two axes recovered by BFS (nearest-neighbour stencils, any
 // row order): part[i] per row, the tile edge and the tile count.
-bool bfs_tiles(int n, const int *ai, const int *aj, int max_parts, int max_rows,
-               std::vector<int> &part, int &tau, int &nparts, std::string &why) {
+//
+// The tile edge: the smallest power of two whose tile count fits the resident
+// workgroups, then doubled while a tile's rows of one level still fit one
+// group (the solve takes as long over a group of 64 rows as over one of 8, and
+// every tile on the way costs a hand-over), at least kMinTiles tiles remain
+// and a tile's faces stay small (kMaxFace rows of other tiles). Measured per
+// apply, smallest edge -> this rule: 128^2 5-point IC(0) FP64 (256 -> 4 tiles)
+// 171 -> 122 us, 512^2 (256 -> 64 tiles) 372 -> 364 us.
+constexpr int kMinTiles = 4;
+constexpr int kMaxFace = 8192;
+bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes, int max_parts,
+               int max_rows, std::vector<int> &part, int &tau, int &nparts, std::string &why) {
   const int64_t nnz = ai[n];
   // symmetric adjacency of the triangle (T + T^T)
   std::vector<int> ptr(static_cast<size_t>(n) + 1, 0), adj(static_cast<size_t>(2 * nnz));
@@ -214,30 +224,60 @@ bool bfs_tiles(int n, const int *ai, const int *aj, int max_parts, int max_rows,
   }
   const int umax = *std::max_element(u.begin(), u.end());
   const int vmax = *std::max_element(v.begin(), v.end());
-  // the smallest square tile whose count fits the resident workgroups and
-  // whose rows fit LDS
   part.assign(static_cast<size_t>(n), 0);
   tau = 0;
   nparts = 0;
+  auto tile_of = [&](int i, int t, int nv) {
+    return static_cast<size_t>(u[i] / t) * nv + v[i] / t;
+  };
+  std::vector<int> by_level;  // rows level by level, when a larger edge is tried
   for (int t = 2; t <= 4096; t *= 2) {
     const int nu = umax / t + 1, nv = vmax / t + 1;
     if (static_cast<int64_t>(nu) * nv > 4 * static_cast<int64_t>(max_parts)) continue;
     std::vector<int> cnt(static_cast<size_t>(nu) * nv, 0);
-    for (int i = 0; i < n; ++i) cnt[static_cast<size_t>(u[i] / t) * nv + v[i] / t]++;
+    for (int i = 0; i < n; ++i) cnt[tile_of(i, t, nv)]++;
     int used = 0, big = 0;
     for (int c : cnt) {
       used += c > 0;
       big = std::max(big, c);
     }
-    if (used <= max_parts && big <= max_rows) {
-      std::vector<int> id(cnt.size(), -1);
-      nparts = 0;
-      for (size_t c = 0; c < cnt.size(); ++c)
-        if (cnt[c]) id[c] = nparts++;
-      for (int i = 0; i < n; ++i) part[i] = id[static_cast<size_t>(u[i] / t) * nv + v[i] / t];
-      tau = t;
-      break;
+    if (used > max_parts || big > max_rows) {
+      if (tau) break;
+      continue;
     }
+    if (tau) {
+      // a larger edge: one group per level, tiles and faces as above
+      if (used < kMinTiles) break;
+      if (by_level.empty()) {
+        int top = 0;
+        for (int i = 0; i < n; ++i) top = std::max(top, level[i]);
+        std::vector<int> at(static_cast<size_t>(top) + 2, 0);
+        for (int i = 0; i < n; ++i) at[level[i] + 1]++;
+        for (int l = 0; l <= top; ++l) at[l + 1] += at[l];
+        by_level.resize(static_cast<size_t>(n));
+        for (int i = 0; i < n; ++i) by_level[at[level[i]]++] = i;
+      }
+      std::vector<int> seen(cnt.size(), -1), rows(cnt.size(), 0), face(cnt.size(), 0);
+      bool fits = true;
+      for (int k = 0; k < n && fits; ++k) {
+        const int i = by_level[k];
+        const size_t c = tile_of(i, t, nv);
+        if (seen[c] != level[i]) {
+          seen[c] = level[i];
+          rows[c] = 0;
+        }
+        fits = ++rows[c] <= lanes;
+        for (int q = ai[i]; q < ai[i + 1]; ++q) face[c] += tile_of(aj[q], t, nv) != c;
+        fits = fits && face[c] <= kMaxFace;
+      }
+      if (!fits) break;
+    }
+    std::vector<int> id(cnt.size(), -1);
+    nparts = 0;
+    for (size_t c = 0; c < cnt.size(); ++c)
+      if (cnt[c]) id[c] = nparts++;
+    for (int i = 0; i < n; ++i) part[i] = id[tile_of(i, t, nv)];
+    tau = t;
   }
   if (!tau) {
     why = "no tile size fits";
@@ -263,7 +303,8 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
   int tau = 0, nparts = 0, rl = 1;
   bool box = false;
   if (maxe <= kTileMaxEntries) {
-    if (!bfs_tiles(n, ai, aj, max_parts, max_rows, part, tau, nparts, why)) return false;
+    if (!bfs_tiles(n, ai, aj, level, lanes, max_parts, max_rows, part, tau, nparts, why))
+      return false;
   } else if (maxe <= kTileRowLanes * kTileMaxEntries) {
     int nx = 0, ny = 0, nz = 0;
     if (!detect_box_grid(n, ai, aj, nx, ny, nz)) {

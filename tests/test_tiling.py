@@ -212,3 +212,24 @@ def test_tiled_layout_refusals(tl):
     L, _, _ = orc.split_ldu(S)
     ok, why, _, _ = _build(tl, L, False)
     assert not ok and "few" in why
+
+
+@pytest.mark.parametrize("dims,most", [((128, 128), 64), ((128, 130), 64), ((200, 40), 64),
+                                       ((34, 33, 40), 64), ((17, 70, 9), 64), ((20, 20, 20), 64)])
+def test_tile_edge_rule(tl, dims, most):
+    """Grids on both sides of the tile-edge rule: tiles are enlarged only
+    while the rows of one level in a tile fit one group, at least four tiles
+    remain, and the layout still replays to plain substitution."""
+    A = la.gen.poisson2d(*dims) if len(dims) == 2 else la.gen.laplace3d(*dims)
+    F = orc.iluk(_o(_rcm(A) if dims == (20, 20, 20) else A), 0)[0]
+    L, D, U = orc.split_ldu(F)
+    b = la.gen.uniform(F.n, 23)
+    for T, diag, upper, ref in ((L, None, False, orc.forward_sub(L, b)),
+                                (U, D, True, orc.backward_sub(U, D, b))):
+        x, nparts, rl = _replay(tl, T, diag, b, upper)
+        assert 4 <= nparts <= 256 and rl == 1
+        assert np.abs(x - ref).max() <= 1e-12 * np.abs(ref).max()
+        v = np.zeros(7, np.int32)
+        tl.tiling_sizes(_p(v))
+        lv = _levels(T.n, np.asarray(T.ai), np.asarray(T.aj), upper)
+        assert v[1] <= nparts * (lv.max() + 1)  # one group per level and tile
