@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstdlib>
+#include <type_traits>
 
 #include "dev_util.hpp"
 #include "device.hpp"
@@ -267,15 +268,23 @@ __device__ __forceinline__ void lds_store(int *p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// A group's packed record: E values, E byte addresses into LDS (32-bit) and
-// 1/d per lane. Values and addresses are cut into pieces of at most 16 bytes
-// per lane, piece by piece for all 64 lanes, so that every load covers one
-// contiguous run.
+// A group's packed record: E values, E LDS addresses and 1/d per lane. Values
+// and addresses are cut into pieces of at most 16 bytes per lane, piece by
+// piece for all 64 lanes, so that every load covers one contiguous run. An
+// address is a byte address in 32 bits, ready to use; eight FP64 values leave
+// no registers for that at kTileDepth groups (256 are all a wavefront of
+// these workgroups gets), so there it is a slot number in 16 bits (27-point
+// ILU(1) on 90^3, FP64: 921 -> 762 us per apply, without spilled registers).
 template <int E, typename T>
 struct TileRec {
+  static constexpr bool kWide = !(E == 8 && sizeof(T) == 8);
+  using Code = std::conditional_t<kWide, uint32_t, uint16_t>;
+  // from an LDS byte address
+  static __host__ __device__ Code code(int a) { return static_cast<Code>(kWide ? a : a / 8); }
+  static __device__ uint32_t address(Code c) { return kWide ? c : static_cast<uint32_t>(c) * 8u; }
   static constexpr int kVal = E * static_cast<int>(sizeof(T));
   static constexpr int kValPiece = kVal < 16 ? kVal : 16;
-  static constexpr int kCode = E * 4;
+  static constexpr int kCode = E * static_cast<int>(sizeof(Code));
   static constexpr int kCodePiece = 16;
   static constexpr int kCodeAt = kTileLanes * kVal;
   static constexpr int kDinvAt = kCodeAt + kTileLanes * kCode;
@@ -315,7 +324,7 @@ __device__ __forceinline__ double tile_val(double v) { return v; }
 // one pipeline stage: a group's record for this lane
 template <int E, typename T>
 struct TileStage {
-  alignas(16) uint32_t code[E];
+  alignas(16) typename TileRec<E, T>::Code code[E];
   alignas(16) T val[E];
   T dinv;
 };
@@ -419,7 +428,7 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
       auto read_row = [&](const TileStage<E, T> &g, int bpos) {
         bv = bslot(bpos);
 #pragma unroll
-        for (int e = 0; e < E; ++e) xv[e] = *lds_at<V>(g.code[e]);
+        for (int e = 0; e < E; ++e) xv[e] = *lds_at<V>(R::address(g.code[e]));
       };
       if (nblk > 0 && !tile_wait(&s_b[0], 0)) s_late = 1;
       lds_fence();
@@ -695,11 +704,12 @@ __global__ void k_tile_pack(int64_t slots, const int *__restrict__ src,
   for (int e = 0; e < E; ++e) {
     const int q = src[t * E + e];
     constexpr int sT = static_cast<int>(sizeof(T));
-    const int vb = e * sT, cb = e * 4;
+    const int vb = e * sT, cb = e * static_cast<int>(sizeof(typename R::Code));
     *reinterpret_cast<T *>(rec + vb / R::kValPiece * R::kValPiece * kTileLanes +
                            lane * R::kValPiece + vb % R::kValPiece) = q >= 0 ? val[q] : T();
-    *reinterpret_cast<int *>(rec + R::kCodeAt + cb / R::kCodePiece * R::kCodePiece * kTileLanes +
-                             lane * R::kCodePiece + cb % R::kCodePiece) = code[t * E + e];
+    *reinterpret_cast<typename R::Code *>(
+        rec + R::kCodeAt + cb / R::kCodePiece * R::kCodePiece * kTileLanes +
+        lane * R::kCodePiece + cb % R::kCodePiece) = R::code(code[t * E + e]);
   }
   T d = T();
   if (dinv && dpos[t] >= 0) d = dinv[dpos[t]];
