@@ -438,7 +438,7 @@ int la_trsv_solve(la_trsv_t T, la_trsv_mode mode, la_dtype val, la_dtype vec, co
   LA_TRY
   LA_CHECK_ARG(T, "null handle");
   trsv_solve(*T->t, mode, val, vec, b, x, T->t->stream);
-  if (mode == LA_TRSV_SYNCFREE && trsv_check_timeout(*T->t, T->t->stream))
+  if (mode == LA_TRSV_SYNCFREE && trsv_check_timeout({T->t.get()}, T->t->stream))
     throw la_error(LA_ERR_TIMEOUT, "sync-free triangular solve exceeded its spin bound");
   LA_CATCH
 }
@@ -448,7 +448,7 @@ int la_trsv_solve_transpose(la_trsv_t T, la_trsv_mode mode, la_dtype val, la_dty
   LA_CHECK_ARG(T, "null handle");
   TrsvPlan &Tt = trsv_transposed(*T->t);
   trsv_solve(Tt, mode, val, vec, b, x, T->t->stream);
-  if (mode == LA_TRSV_SYNCFREE && trsv_check_timeout(Tt, T->t->stream))
+  if (mode == LA_TRSV_SYNCFREE && trsv_check_timeout({&Tt}, T->t->stream))
     throw la_error(LA_ERR_TIMEOUT, "sync-free triangular solve exceeded its spin bound");
   LA_CATCH
 }
@@ -545,8 +545,8 @@ int la_prec_apply(la_prec_t P, la_trsv_mode mode, la_dtype val, la_dtype vec, co
   LA_TRY
   LA_CHECK_ARG(P, "null handle");
   prec_apply(*P->p, mode, val, vec, r, z, P->p->stream);
-  if (mode == LA_TRSV_SYNCFREE && (trsv_check_timeout(*P->p->lower, P->p->stream) ||
-                                   trsv_check_timeout(*P->p->upper, P->p->stream)))
+  if (mode == LA_TRSV_SYNCFREE &&
+      trsv_check_timeout({P->p->lower.get(), P->p->upper.get()}, P->p->stream))
     throw la_error(LA_ERR_TIMEOUT, "sync-free triangular solve exceeded its spin bound");
   LA_CATCH
 }

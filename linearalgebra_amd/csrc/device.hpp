@@ -1,6 +1,7 @@
 // Device-side objects of the hot path (matrix, triangular-solve plan,
 // preconditioner) and the launchers the host code calls.
 #pragma once
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <string>
@@ -93,7 +94,11 @@ struct TrsvPlan {
   MultiValues val, diag;       // values / reciprocal diagonal in level order
   std::vector<int> level_ptr;  // host, nlevels+1
   int nchunks = 0;
-  DevBuf chunk_start, counter, err_flag;
+  DevBuf chunk_start, counter;
+  // a wait ran out of time: the device's flag, with the address of the host's
+  // copy (coherent pinned memory) behind it
+  DevBuf err_flag;
+  int *err_host = nullptr;
   // sync-free launch shape: confined to one XCD (plain stores, L2-latency
   // polls) or spread over all XCDs; workgroups taking part
   bool sf_xlocal = true;
@@ -166,8 +171,9 @@ void trsv_set_sources(TrsvPlan &T, const int64_t *src, const int64_t *dsrc, hipS
 void trsv_refresh(TrsvPlan &T, const double *f, hipStream_t s);
 // JACOBI mode sweep count for T and its transposed plan (0..1000000)
 void trsv_set_sweeps(TrsvPlan &T, int sweeps);
-// checks (and clears) the sync-free spin-bound error flag; synchronizes s
-bool trsv_check_timeout(TrsvPlan &T, hipStream_t s);
+// synchronizes s, then checks (and clears) the sync-free spin-bound error
+// flags of the plans and their transposed plans
+bool trsv_check_timeout(std::initializer_list<TrsvPlan *> plans, hipStream_t s);
 
 // -------------------------------------------------------------- ILU / IC
 struct NumericPlan;

@@ -446,7 +446,7 @@ int run_solver(Mat &A, Prec *P, const la_solver_opts &o, const double *b, double
       !(out.rel_residual < o.rel_tol || tr < o.abs_tol * 1.0000001))
     out.converged = 0;  // recurrence said yes, the true residual says no
   for (Prec *Q : {P, tl_right}) {
-    if (Q && (trsv_check_timeout(*Q->lower, s) || trsv_check_timeout(*Q->upper, s)))
+    if (Q && trsv_check_timeout({Q->lower.get(), Q->upper.get()}, s))
       throw la_error(LA_ERR_TIMEOUT, "sync-free triangular solve exceeded its spin bound");
   }
   if (res) *res = out;

@@ -104,6 +104,14 @@ __global__ void k_fill_sentinel(int64_t n, V *x, unsigned *ctl) {
 // every 256 polls and gives up too, so the kernel always drains quickly.
 constexpr uint64_t kWaitTicks = 20000000;  // 0.2 s
 
+// a wait ran out of time: *err for the polling wavefronts, and the host's copy
+// (its address sits behind the flag), which trsv_check_timeout reads
+__device__ __forceinline__ void flag_late(int *err) {
+  __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  int *const host = *reinterpret_cast<int *const *>(err + 2);
+  __hip_atomic_store(host, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // One row of a sync-free solve, G lanes: wait for each x_j, accumulate,
 // publish x_r. `sub` is the lane's index inside its group.
 template <int G, typename T, typename V, typename A, bool DIAG, bool XLOCAL>
@@ -144,7 +152,7 @@ __device__ __forceinline__ void sf_row(int k, int sub, const int *__restrict__ r
     }
     acc += a * A(is_sentinel(xv) ? V(0) : xv);
   }
-  if (gave_up) __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (gave_up) flag_late(err);
   acc = group_sum<G>(acc);
   if (sub == 0) {
     A v = bb - acc;
@@ -271,13 +279,14 @@ __device__ __forceinline__ void lds_store(int *p, int v) {
 // A group's packed record: E values, E LDS addresses and 1/d per lane. Values
 // and addresses are cut into pieces of at most 16 bytes per lane, piece by
 // piece for all 64 lanes, so that every load covers one contiguous run. An
-// address is a byte address in 32 bits, ready to use; eight FP64 values leave
-// no registers for that at kTileDepth groups (256 are all a wavefront of
-// these workgroups gets), so there it is a slot number in 16 bits (27-point
-// ILU(1) on 90^3, FP64: 921 -> 762 us per apply, without spilled registers).
+// address is a byte address in 32 bits, ready to use; with eight values per
+// lane it is a slot number in 16 bits, which takes half the registers (eight
+// FP64 values at kTileDepth groups spilled otherwise: 256 are all a wavefront
+// of these workgroups gets) and one load less (27-point ILU(1) per apply: 90^3
+// FP64 921 -> 762 us, 56^3 FP32 451 -> 438 us).
 template <int E, typename T>
 struct TileRec {
-  static constexpr bool kWide = !(E == 8 && sizeof(T) == 8);
+  static constexpr bool kWide = E < 8;
   using Code = std::conditional_t<kWide, uint32_t, uint16_t>;
   // from an LDS byte address
   static __host__ __device__ Code code(int a) { return static_cast<Code>(kWide ? a : a / 8); }
@@ -527,7 +536,7 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
             if ((polls & 255u) == 0 &&
                 (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
                  __builtin_amdgcn_s_memrealtime() - w0 > kWaitTicks)) {
-              __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              flag_late(err);
               if (pending) slot(e.y) = V(0);
               break;
             }
@@ -623,8 +632,7 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
       }
     }
     // a wait of the solver that ran out of time
-    if (wave == 0 && s_late && lane == 0)
-      __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (wave == 0 && s_late && lane == 0) flag_late(err);
     __syncthreads();
   }
 }
@@ -1116,6 +1124,7 @@ hipStream_t capture_stream() {
 }  // namespace
 
 TrsvPlan::~TrsvPlan() {
+  if (err_host) (void)hipHostFree(err_host);
   for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
 }
 
@@ -1210,7 +1219,16 @@ std::unique_ptr<TrsvPlan> make_trsv(int n, int base, const int *ai, const int *a
   P->col.upload(cl.data(), sizeof(int) * nnz, s);
   P->perm.upload(iperm.data(), sizeof(int) * n, s);
   P->chunk_start.upload(chunks.data(), sizeof(int) * chunks.size(), s);
-  LA_HIP(hipMemsetAsync(P->err_flag.p, 0, sizeof(int) * 4, s));
+  LA_HIP(hipHostMalloc(reinterpret_cast<void **>(&P->err_host), sizeof(int) * 4,
+                       hipHostMallocMapped | hipHostMallocCoherent));
+  *P->err_host = 0;
+  struct {
+    int flag[2];
+    int *host;
+  } flag = {{0, 0}, nullptr};
+  static_assert(sizeof(flag) == sizeof(int) * 4, "the host copy's address behind the flag");
+  LA_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&flag.host), P->err_host, 0));
+  P->err_flag.upload(&flag, sizeof(flag), s);
   LA_HIP(hipMemsetAsync(P->counter.p, 0, sizeof(unsigned) * 16, s));
   P->val.set_from_host(vl.data(), nnz, s);
   if (diag) P->diag.set_from_host(dg.data(), n, s);
@@ -1364,13 +1382,20 @@ void trsv_set_sweeps(TrsvPlan &T, int sweeps) {
   if (T.transposed) trsv_set_sweeps(*T.transposed, sweeps);
 }
 
-bool trsv_check_timeout(TrsvPlan &T, hipStream_t s) {
-  int flag = 0;
-  LA_HIP(hipMemcpyAsync(&flag, T.err_flag.p, sizeof(int), hipMemcpyDeviceToHost, s));
+// The flag reaches the host as a store of the kernel that set it, so one
+// synchronisation is all a check costs (a copy of the flag and another
+// synchronisation per triangle took 35 us more per apply).
+bool trsv_check_timeout(std::initializer_list<TrsvPlan *> plans, hipStream_t s) {
   LA_HIP(hipStreamSynchronize(s));
-  if (flag) LA_HIP(hipMemsetAsync(T.err_flag.p, 0, sizeof(int), s));
-  bool bad = flag != 0;
-  if (T.transposed) bad = trsv_check_timeout(*T.transposed, s) || bad;
+  bool bad = false;
+  for (TrsvPlan *T : plans)
+    for (; T; T = T->transposed.get())
+      if (__atomic_load_n(T->err_host, __ATOMIC_ACQUIRE) != 0) {
+        bad = true;
+        LA_HIP(hipMemsetAsync(T->err_flag.p, 0, sizeof(int), s));
+        LA_HIP(hipStreamSynchronize(s));
+        __atomic_store_n(T->err_host, 0, __ATOMIC_RELEASE);
+      }
   return bad;
 }
 
