@@ -61,25 +61,6 @@ __global__ void k_reduce_partials(int k, int nb, const double *__restrict__ part
 }
 
 template <typename V>
-__global__ __launch_bounds__(kB) void k_multidot_partial(int64_t n, int k,
-                                                         const V *__restrict__ Vm, int64_t ld,
-                                                         const V *__restrict__ w,
-                                                         double *part) {
-  __shared__ double sh[kB / 64];
-  // one pass per basis vector; w is re-read from L2
-  for (int i = 0; i < k; ++i) {
-    const V *v = Vm + static_cast<int64_t>(i) * ld;
-    double acc = 0;
-    for (int64_t t = static_cast<int64_t>(blockIdx.x) * kB + threadIdx.x; t < n;
-         t += static_cast<int64_t>(gridDim.x) * kB)
-      acc += static_cast<double>(v[t]) * static_cast<double>(w[t]);
-    const double s = block_reduce<V>(acc, sh);
-    if (threadIdx.x == 0) part[static_cast<int64_t>(i) * gridDim.x + blockIdx.x] = s;
-    __syncthreads();
-  }
-}
-
-template <typename V>
 __global__ __launch_bounds__(kB) void k_multiaxpy(int64_t n, int k, const V *__restrict__ Vm,
                                                   int64_t ld, const double *__restrict__ h,
                                                   V *w) {
@@ -243,6 +224,137 @@ __global__ __launch_bounds__(kB) void k_multiaxpy_v(int64_t n, int k, const V *_
     for (int i = 0; i < k; ++i) acc -= h[i] * static_cast<double>(Vm[static_cast<int64_t>(i) * ld + t]);
     w[t] = static_cast<V>(acc);
   }
+}
+
+// One Gram-Schmidt step of k <= KM basis vectors: w -= sum_i h_i V_i (the
+// arithmetic of k_multiaxpy_v) and, from the same registers, the next pass's
+// dot products <V_i, w> (grid and partials of k_multidot_partial_v; FP64:
+// the same sums bit for bit). Bound by the basis' bytes, which the two kernels
+// read twice: a thread keeps its two values of every V_i (KM loads in flight,
+// 4 KM registers as FP64) and KM FP64 sums; two workgroups a CU, the grid's
+// size, leave 256 registers a lane, so KM ends at kGsFused = 32 and FP32 takes
+// 8-byte loads (four values of each spill: 25 vectors of 1M rows 7 % slower
+// than two passes). With k_gs_update_norm, 25 unpreconditioned steps of 1M
+// rows: 3.15 -> 2.75 ms, FP32 2.36 -> 2.25 ms.
+constexpr int kGsFused = 32;
+template <int KM, typename V>
+__global__ __launch_bounds__(kB, 2) void k_gs_update_dots(int64_t n, int k,
+                                                          const V *__restrict__ Vm, int64_t ld,
+                                                          const double *__restrict__ h, V *w,
+                                                          double *part) {
+  using T = std::conditional_t<std::is_same_v<V, double>, double2, float2>;
+  constexpr int K = 2;
+  __shared__ double sh[KM][kB / 64];
+  T *wv = reinterpret_cast<T *>(w);
+  const int64_t nv = n / K, stride = static_cast<int64_t>(gridDim.x) * kB;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double dot[KM];
+#pragma unroll
+  for (int i = 0; i < KM; ++i) dot[i] = 0;
+  for (int64_t v = static_cast<int64_t>(blockIdx.x) * kB + threadIdx.x; v < nv; v += stride) {
+    T b = wv[v];
+    T a[KM];
+#pragma unroll
+    for (int i = 0; i < KM; ++i)
+      if (i < k) a[i] = reinterpret_cast<const T *>(Vm + static_cast<int64_t>(i) * ld)[v];
+    double acc[K];
+#pragma unroll
+    for (int c = 0; c < K; ++c) acc[c] = static_cast<double>(vel<T, V>(b, c));
+#pragma unroll
+    for (int i = 0; i < KM; ++i)
+      if (i < k) {
+        const double hi = h[i];
+#pragma unroll
+        for (int c = 0; c < K; ++c) acc[c] -= hi * static_cast<double>(vel<T, V>(a[i], c));
+      }
+#pragma unroll
+    for (int c = 0; c < K; ++c) vel<T, V>(b, c) = static_cast<V>(acc[c]);
+    wv[v] = b;
+#pragma unroll
+    for (int i = 0; i < KM; ++i)
+      if (i < k)
+#pragma unroll
+        for (int c = 0; c < K; ++c)
+          dot[i] += static_cast<double>(vel<T, V>(a[i], c)) * static_cast<double>(vel<T, V>(b, c));
+  }
+  if (blockIdx.x == 0 && threadIdx.x < n - nv * K) {
+    const int64_t t = nv * K + threadIdx.x;
+    double acc = static_cast<double>(w[t]);
+    for (int i = 0; i < k; ++i)
+      acc -= h[i] * static_cast<double>(Vm[static_cast<int64_t>(i) * ld + t]);
+    const V wt = static_cast<V>(acc);
+    w[t] = wt;
+#pragma unroll
+    for (int i = 0; i < KM; ++i)
+      if (i < k)
+        dot[i] += static_cast<double>(Vm[static_cast<int64_t>(i) * ld + t]) *
+                  static_cast<double>(wt);
+  }
+#pragma unroll
+  for (int i = 0; i < KM; ++i)
+    if (i < k) {
+      const double t = wave_sum(dot[i]);
+      if (lane == 0) sh[i][wave] = t;
+    }
+  __syncthreads();
+  if (threadIdx.x < k) {
+    double t = 0;
+    for (int q = 0; q < kB / 64; ++q) t += sh[threadIdx.x][q];
+    part[static_cast<int64_t>(threadIdx.x) * gridDim.x + blockIdx.x] = t;
+  }
+}
+
+// w -= sum_i h_i V_i and the partial sums of <w, w> (those of
+// k_dot_partial_v, bit for bit): the norm costs no pass of its own over w, and
+// kMdG loads are in flight.
+template <typename V>
+__global__ __launch_bounds__(kB) void k_gs_update_norm(int64_t n, int k,
+                                                       const V *__restrict__ Vm, int64_t ld,
+                                                       const double *__restrict__ h, V *w,
+                                                       double *part) {
+  using T = typename V16<V>::T;
+  constexpr int K = V16<V>::k;
+  __shared__ double sh[kB / 64];
+  T *wv = reinterpret_cast<T *>(w);
+  const int64_t nv = n / K, stride = static_cast<int64_t>(gridDim.x) * kB;
+  double dot = 0;
+  for (int64_t v = static_cast<int64_t>(blockIdx.x) * kB + threadIdx.x; v < nv; v += stride) {
+    T b = wv[v];
+    double acc[K];
+#pragma unroll
+    for (int c = 0; c < K; ++c) acc[c] = static_cast<double>(vel<T, V>(b, c));
+    for (int i0 = 0; i0 < k; i0 += kMdG) {
+      T a[kMdG];
+#pragma unroll
+      for (int e = 0; e < kMdG; ++e)
+        if (i0 + e < k)
+          a[e] = reinterpret_cast<const T *>(Vm + static_cast<int64_t>(i0 + e) * ld)[v];
+#pragma unroll
+      for (int e = 0; e < kMdG; ++e)
+        if (i0 + e < k) {
+          const double hi = h[i0 + e];
+#pragma unroll
+          for (int c = 0; c < K; ++c) acc[c] -= hi * static_cast<double>(vel<T, V>(a[e], c));
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      vel<T, V>(b, c) = static_cast<V>(acc[c]);
+      dot += static_cast<double>(vel<T, V>(b, c)) * static_cast<double>(vel<T, V>(b, c));
+    }
+    wv[v] = b;
+  }
+  if (blockIdx.x == 0 && threadIdx.x < n - nv * K) {
+    const int64_t t = nv * K + threadIdx.x;
+    double acc = static_cast<double>(w[t]);
+    for (int i = 0; i < k; ++i)
+      acc -= h[i] * static_cast<double>(Vm[static_cast<int64_t>(i) * ld + t]);
+    const V wt = static_cast<V>(acc);
+    w[t] = wt;
+    dot += static_cast<double>(wt) * static_cast<double>(wt);
+  }
+  const double t = block_reduce<V>(dot, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
 template <typename V>
@@ -651,22 +763,25 @@ void dot_dev(int64_t n, la_dtype vec, const void *x, const void *y, double *part
   LA_HIP(hipGetLastError());
 }
 
+namespace {
+// the Gram-Schmidt kernels take 16-byte loads: the solver's bases are padded
+// to whole 16-byte rows
+void check_basis(la_dtype vec, const void *V, int64_t ld, const void *w) {
+  const size_t es = vec == LA_F64 ? sizeof(double) : sizeof(float);
+  LA_CHECK_ARG(al16(V) && al16(w) && (static_cast<size_t>(ld) * es) % 16 == 0,
+               "basis vectors not 16-byte aligned");
+}
+}  // namespace
+
 void multidot_dev(int64_t n, int k, la_dtype vec, const void *V, int64_t ld, const void *w,
                   double *partials, double *out, hipStream_t s) {
   LA_CHECK_ARG(k <= kMaxDots, "too many dot products");
-  const size_t es = vec == LA_F64 ? sizeof(double) : sizeof(float);
-  const bool v16 = al16(V) && al16(w) && (static_cast<size_t>(ld) * es) % 16 == 0;
-  if (vec == LA_F64 && v16)
+  check_basis(vec, V, ld, w);
+  if (vec == LA_F64)
     hipLaunchKernelGGL(k_multidot_partial_v<double>, dim3(kRedBlocks), dim3(kB), 0, s, n, k,
                        static_cast<const double *>(V), ld, static_cast<const double *>(w), partials);
-  else if (v16)
-    hipLaunchKernelGGL(k_multidot_partial_v<float>, dim3(kRedBlocks), dim3(kB), 0, s, n, k,
-                       static_cast<const float *>(V), ld, static_cast<const float *>(w), partials);
-  else if (vec == LA_F64)
-    hipLaunchKernelGGL(k_multidot_partial<double>, dim3(kRedBlocks), dim3(kB), 0, s, n, k,
-                       static_cast<const double *>(V), ld, static_cast<const double *>(w), partials);
   else
-    hipLaunchKernelGGL(k_multidot_partial<float>, dim3(kRedBlocks), dim3(kB), 0, s, n, k,
+    hipLaunchKernelGGL(k_multidot_partial_v<float>, dim3(kRedBlocks), dim3(kB), 0, s, n, k,
                        static_cast<const float *>(V), ld, static_cast<const float *>(w), partials);
   LA_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_reduce_partials, dim3(std::max(k, 1)), dim3(kB), 0, s, k, kRedBlocks,
@@ -693,6 +808,56 @@ void multiaxpy_dev(int64_t n, int k, la_dtype vec, const void *V, int64_t ld, co
   else
     hipLaunchKernelGGL(k_multiaxpy<float>, dim3(grid_for(n)), dim3(kB), 0, s, n, k,
                        static_cast<const float *>(V), ld, h, static_cast<float *>(w));
+  LA_HIP(hipGetLastError());
+}
+
+namespace {
+template <typename V>
+void launch_update_dots(int64_t n, int k, const void *Vm, int64_t ld, const double *h, void *w,
+                        double *partials, hipStream_t s) {
+  const V *v = static_cast<const V *>(Vm);
+  auto kern = k <= 8    ? k_gs_update_dots<8, V>
+              : k <= 16 ? k_gs_update_dots<16, V>
+              : k <= 24 ? k_gs_update_dots<24, V>
+                        : k_gs_update_dots<kGsFused, V>;
+  hipLaunchKernelGGL(kern, dim3(kRedBlocks), dim3(kB), 0, s, n, k, v, ld, h, static_cast<V *>(w),
+                     partials);
+  LA_HIP(hipGetLastError());
+}
+}  // namespace
+
+void update_dots_dev(int64_t n, int k, la_dtype vec, const void *V, int64_t ld, const double *h,
+                     void *w, double *partials, double *out, hipStream_t s) {
+  const size_t es = vec == LA_F64 ? sizeof(double) : sizeof(float);
+  check_basis(vec, V, ld, w);
+  if (k > kGsFused) {  // more than the registers hold: two passes
+    for (int c0 = 0; c0 < k; c0 += kMaxDots)
+      multiaxpy_dev(n, std::min(kMaxDots, k - c0), vec,
+                    static_cast<const char *>(V) + es * static_cast<size_t>(ld) * c0, ld, h + c0,
+                    w, s);
+    for (int c0 = 0; c0 < k; c0 += kMaxDots)
+      multidot_dev(n, std::min(kMaxDots, k - c0), vec,
+                   static_cast<const char *>(V) + es * static_cast<size_t>(ld) * c0, ld, w,
+                   partials, out + c0, s);
+    return;
+  }
+  if (vec == LA_F64) launch_update_dots<double>(n, k, V, ld, h, w, partials, s);
+  else launch_update_dots<float>(n, k, V, ld, h, w, partials, s);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(k), dim3(kB), 0, s, k, kRedBlocks, partials, out);
+  LA_HIP(hipGetLastError());
+}
+
+void update_norm_dev(int64_t n, int k, la_dtype vec, const void *V, int64_t ld, const double *h,
+                     void *w, double *partials, double *out, hipStream_t s) {
+  check_basis(vec, V, ld, w);
+  if (vec == LA_F64)
+    hipLaunchKernelGGL(k_gs_update_norm<double>, dim3(kRedBlocks), dim3(kB), 0, s, n, k,
+                       static_cast<const double *>(V), ld, h, static_cast<double *>(w), partials);
+  else
+    hipLaunchKernelGGL(k_gs_update_norm<float>, dim3(kRedBlocks), dim3(kB), 0, s, n, k,
+                       static_cast<const float *>(V), ld, h, static_cast<float *>(w), partials);
+  LA_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kB), 0, s, 1, kRedBlocks, partials, out);
   LA_HIP(hipGetLastError());
 }
 

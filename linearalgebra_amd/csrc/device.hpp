@@ -247,12 +247,19 @@ void dot_dev(int64_t n, la_dtype vec, const void *x, const void *y, double *part
 // allocation; calls that overlap on one GPU share that array and race
 void dot_noalloc(int64_t n, la_dtype vec, const void *x, const void *y, double *out_dev,
                  hipStream_t s);
-// out[i] = <V_i, w> for i < k; V is k vectors of length n, stride ld
+// out[i] = <V_i, w> for i < k; V is k vectors of length n, stride ld (here and
+// in update_*_dev: V, w and every V_i 16-byte aligned)
 void multidot_dev(int64_t n, int k, la_dtype vec, const void *V, int64_t ld, const void *w,
                   double *partials, double *out, hipStream_t s);
 // w -= sum_i h[i] V_i (h device FP64)
 void multiaxpy_dev(int64_t n, int k, la_dtype vec, const void *V, int64_t ld, const double *h,
                    void *w, hipStream_t s);
+// w -= sum_i h[i] V_i, then out[i] = <V_i, w> (any k)
+void update_dots_dev(int64_t n, int k, la_dtype vec, const void *V, int64_t ld, const double *h,
+                     void *w, double *partials, double *out, hipStream_t s);
+// w -= sum_i h[i] V_i, then out[0] = <w, w> (any k)
+void update_norm_dev(int64_t n, int k, la_dtype vec, const void *V, int64_t ld, const double *h,
+                     void *w, double *partials, double *out, hipStream_t s);
 // y = a*x + b*y with host scalars
 void axpby(int64_t n, la_dtype vec, double a, const void *x, double b, void *y,
            hipStream_t s);

@@ -193,15 +193,16 @@ CgResult fgmres_core(Mat &A, Prec *P, const la_solver_opts &o, la_dtype val, la_
   const int64_t n = A.rows;
   const la_dtype acc = (val == LA_F64 && vec == LA_F64) ? LA_F64 : LA_F32;
   const size_t es = dtype_size(vec);
+  const int64_t ld = (n + 3) / 4 * 4;  // every basis vector 16-byte aligned
   if (W.m < m || W.basis_dt != vec || !W.V.p) {
-    W.V.alloc(es * static_cast<size_t>(n) * (m + 1));
-    W.Z.alloc(es * static_cast<size_t>(n) * m);
+    W.V.alloc(es * static_cast<size_t>(ld) * (m + 1));
+    W.Z.alloc(es * static_cast<size_t>(ld) * m);
     W.m = m;
     W.basis_dt = vec;
   }
   char *V = static_cast<char *>(W.V.p), *Z = static_cast<char *>(W.Z.p);
-  auto Vj = [&](int j) { return static_cast<void *>(V + es * static_cast<size_t>(n) * j); };
-  auto Zj = [&](int j) { return static_cast<void *>(Z + es * static_cast<size_t>(n) * j); };
+  auto Vj = [&](int j) { return static_cast<void *>(V + es * static_cast<size_t>(ld) * j); };
+  auto Zj = [&](int j) { return static_cast<void *>(Z + es * static_cast<size_t>(ld) * j); };
   DevBuf *vb = vec == LA_F64 ? W.v64 : W.v32;
   void *w = vb[0].p;
   double *part = W.sc.partials.as<double>();
@@ -215,16 +216,11 @@ CgResult fgmres_core(Mat &A, Prec *P, const la_solver_opts &o, la_dtype val, la_
   // pinned staging for the Hessenberg column and the update coefficients
   // (a pageable buffer would add a staged copy per iteration)
   double *hbuf = W.hpin;
-  // Gram-Schmidt against basis vectors [0, k): the dot products and the
-  // update in groups of at most kMaxDots vectors (one group up to m = 63)
+  // Gram-Schmidt against basis vectors [0, k): the first dot products, in
+  // groups of at most kMaxDots vectors (one group up to m = 63)
   auto gs_dots = [&](int k, double *out) {
     for (int c0 = 0; c0 < k; c0 += kMaxDots)
-      multidot_dev(n, std::min(kMaxDots, k - c0), vec, Vj(c0), n, w, part, out + c0, s);
-  };
-  auto gs_update = [&](char *B, int k, const double *h, void *dst) {
-    for (int c0 = 0; c0 < k; c0 += kMaxDots)
-      multiaxpy_dev(n, std::min(kMaxDots, k - c0), vec, B + es * static_cast<size_t>(n) * c0, n,
-                    h + c0, dst, s);
+      multidot_dev(n, std::min(kMaxDots, k - c0), vec, Vj(c0), ld, w, part, out + c0, s);
   };
   CgResult R;
   int total = 0;
@@ -245,10 +241,8 @@ CgResult fgmres_core(Mat &A, Prec *P, const la_solver_opts &o, la_dtype val, la_
       apply_M(P, o, val, vec, Vj(j), Zj(j), n, s);
       op_apply(A, o, alg, val, vec, acc, 1.0, Zj(j), 0.0, w, w, W, s);
       gs_dots(j + 1, h1);
-      gs_update(V, j + 1, h1, w);
-      gs_dots(j + 1, h2);
-      gs_update(V, j + 1, h2, w);
-      dot_dev(n, vec, w, w, part, hn, s);
+      update_dots_dev(n, j + 1, vec, V, ld, h1, w, part, h2, s);
+      update_norm_dev(n, j + 1, vec, V, ld, h2, w, part, hn, s);
       LA_HIP(hipMemcpyAsync(hbuf, h1, sizeof(double) * (2 * cap + 1), hipMemcpyDeviceToHost, s));
       LA_HIP(hipStreamSynchronize(s));
       for (int i = 0; i <= j; ++i) H[static_cast<size_t>(i) * m + j] = hbuf[i] + hbuf[cap + i];
@@ -285,7 +279,8 @@ CgResult fgmres_core(Mat &A, Prec *P, const la_solver_opts &o, la_dtype val, la_
     // x += Z y  (multiaxpy subtracts, so pass -y)
     for (int l = 0; l < k; ++l) hbuf[l] = -y[l];
     LA_HIP(hipMemcpyAsync(h1, hbuf, sizeof(double) * k, hipMemcpyHostToDevice, s));
-    gs_update(Z, k, h1, x);
+    for (int c0 = 0; c0 < k; c0 += kMaxDots)
+      multiaxpy_dev(n, std::min(kMaxDots, k - c0), vec, Zj(c0), ld, h1 + c0, x, s);
     LA_HIP(hipStreamSynchronize(s));
   }
   R.iters = total;

@@ -251,3 +251,40 @@ def test_fgmres_long_restart(dev, restart):
     assert res["converged"] and res["rel_residual"] < 1.01e-10
     assert abs(res["iters"] - it) <= 3
     assert np.linalg.norm(x.cpu().numpy() - xo) <= 1e-6 * np.linalg.norm(xo)
+
+
+@pytest.mark.parametrize("n", [3, 601, 1024, 263001])
+@pytest.mark.parametrize("steps", [1, 8, 9, 17, 25, 32, 33])
+def test_gram_schmidt_groups(dev, n, steps):
+    """FGMRES steps on both sides of each basis length the Gram-Schmidt
+    kernels are built for (8, 16, 24, 32, two passes above), at sizes with a
+    remainder, without one, and above one pass of the grid (2 x 131072 rows).
+    Gram-Schmidt done twice keeps the basis orthogonal to a few eps, so the
+    iterate carries about steps * eps * cond(A) = 33 * 1.1e-16 * 51 = 2e-13
+    of rounding on either side: 50 times that is allowed. With FP32 vectors
+    the same cycles reach the FP64 tolerance in at most one more cycle for
+    each refinement step, which starts a new one."""
+    import torch
+    ai = np.concatenate([[0], np.cumsum(np.r_[2, np.full(n - 2, 3), 2])]).astype(np.int32)
+    aj = (np.repeat(np.arange(n), np.diff(ai)) +
+          np.concatenate([[0, 1], np.tile([-1, 0, 1], n - 2), [-1, 0]])).astype(np.int32)
+    av = np.choose(aj - np.repeat(np.arange(n), np.diff(ai)) + 1, [-0.9, 2.08, -1.1])
+    A = orc.CSR(n, ai, aj, av)
+    k = min(steps, n - 1)
+    b = la.gen.uniform(n, 8)
+    dA = la.DeviceMatrix(as_lib_csr(A))
+    bd = torch.tensor(b, device=dev)
+    x = torch.zeros(n, dtype=torch.float64, device=dev)
+    res = la.fgmres(dA, None, bd, x, rel_tol=1e-30, restart=k, max_iters=k)
+    xo = orc.fgmres(A, b, restart=k, rel_tol=1e-30, maxiter=k)[0]
+    assert res["iters"] == k
+    assert np.linalg.norm(x.cpu().numpy() - xo) <= 1e-11 * np.linalg.norm(xo)
+    kw = dict(rel_tol=1e-9, restart=k, max_iters=20000)
+    if k < 8 or n > 100000:
+        return  # (one step a cycle converges too slowly to be a small test)
+    full = la.fgmres(dA, None, bd, x.zero_(), **kw)
+    mixed = la.fgmres(dA, None, bd, x.zero_(), precision=la.PREC_MIXED_F32, **kw)
+    r = b - orc.spmv(A, x.cpu().numpy())
+    assert full["converged"] and mixed["converged"]
+    assert mixed["iters"] <= full["iters"] + k * mixed["outer_iters"]
+    assert np.linalg.norm(r) <= 1.01e-9 * np.linalg.norm(b)
