@@ -59,7 +59,7 @@ struct TileLayout {
   int rlanes = 1;  // lanes per row (a row's entries are split in order)
   int m_max = 0;   // rows of the largest tile
   int h_max = 0;   // most values one tile reads from other tiles
-  int maxe = 0;    // entries per lane slot (4 or kTileMaxEntries)
+  int maxe = 0;    // entries per lane slot (2, 4 or kTileMaxEntries)
   int tau = 0;     // tile edge in grid steps
   double remote_frac = 0;  // entries read from another tile
   // most rows of one group that other tiles read; those rows come first in

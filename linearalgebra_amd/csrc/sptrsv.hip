@@ -240,8 +240,10 @@ __global__ __launch_bounds__(NT) void k_trsv_syncfree(
 // issued every access but the polls, and whose tiles polled x: 128^3 7-point
 // IC(0) FP64 425 -> 290 us, FP32 in natural order 631 -> 253 us; 100x96x90
 // FP64 494 -> 200 us; 512^2 FP64 569 -> 372 us; 128^2 225 -> 171 us; 27-point
-// ILU(1) 56^3 FP32 740 -> 447 us, 90^3 FP64 1470 -> 929 us. A group takes the
-// solver 0.12-0.13 us (0.245 us before), and a hand-over about 1 us at the
+// ILU(1) 56^3 FP32 740 -> 447 us, 90^3 FP64 1470 -> 929 us (with larger tiles,
+// smaller records and one synchronisation per apply, 259, 169, 303, 85, 404
+// and 736 us of the FP64 grids and the two boxes now). A group takes the
+// solver 0.12 us (0.245 us before), and a hand-over about 1 us at the
 // median; the chain of hand-overs between tiles and of groups inside them is
 // what bounds the solve now. (With the hand-over slots alone the 3-D solves
 // gained 20-40%, but 512^2 lost 8%: one more store per group on the solver.)
@@ -278,7 +280,12 @@ __device__ __forceinline__ void lds_store(int *p, int v) {
 
 // A group's packed record: E values, E LDS addresses and 1/d per lane. Values
 // and addresses are cut into pieces of at most 16 bytes per lane, piece by
-// piece for all 64 lanes, so that every load covers one contiguous run. An
+// piece for all 64 lanes, so that every load covers one contiguous run. Issuing
+// the loads is a quarter of the solving wavefront's time (128^2, FP64: 273
+// cycles a group, 200-210 without them; the LDS write, read and four
+// multiply-adds take the rest), so with two values per lane 1/d sits in the
+// addresses' piece: two loads a group instead of four (5-point IC(0) per
+// apply, FP64: 128^2 94.4 -> 84.8 us, 512^2 338 -> 303 us). An
 // address is a byte address in 32 bits, ready to use; with eight values per
 // lane it is a slot number in 16 bits, which takes half the registers (eight
 // FP64 values at kTileDepth groups spilled otherwise: 256 are all a wavefront
@@ -296,8 +303,11 @@ struct TileRec {
   static constexpr int kCode = E * static_cast<int>(sizeof(Code));
   static constexpr int kCodePiece = 16;
   static constexpr int kCodeAt = kTileLanes * kVal;
-  static constexpr int kDinvAt = kCodeAt + kTileLanes * kCode;
-  static constexpr int kBytes = kDinvAt + kTileLanes * static_cast<int>(sizeof(T));
+  static constexpr bool kJoined = E == 2;  // 1/d behind the addresses
+  static constexpr int kDinvAt = kCodeAt + (kJoined ? kCode : kTileLanes * kCode);
+  static constexpr int kDinvStep = kJoined ? kCodePiece : static_cast<int>(sizeof(T));
+  static constexpr int kBytes =
+      kCodeAt + kTileLanes * (kJoined ? kCodePiece : kCode + static_cast<int>(sizeof(T)));
   static_assert(kBytes % 128 == 0, "whole cache lines");
 };
 
@@ -307,10 +317,13 @@ typedef unsigned int tile_u4 __attribute__((ext_vector_type(4)));
 // every lane
 template <int total, int piece>
 __device__ __forceinline__ void ld_pieces(const char *base, unsigned lane, void *out) {
-  static_assert(piece == 8 || piece == 16, "piece size");
+  static_assert(piece == 4 || piece == 8 || piece == 16, "piece size");
 #pragma unroll
   for (int q = 0; q < total / piece; ++q) {
-    if constexpr (piece == 16)
+    if constexpr (piece == 4)
+      reinterpret_cast<unsigned *>(out)[q] = __builtin_nontemporal_load(
+          reinterpret_cast<const unsigned *>(base + q * piece * kTileLanes + lane * 4u));
+    else if constexpr (piece == 16)
       reinterpret_cast<tile_u4 *>(out)[q] = __builtin_nontemporal_load(
           reinterpret_cast<const tile_u4 *>(base + q * piece * kTileLanes + lane * 16u));
     else
@@ -333,9 +346,11 @@ __device__ __forceinline__ double tile_val(double v) { return v; }
 // one pipeline stage: a group's record for this lane
 template <int E, typename T>
 struct TileStage {
-  alignas(16) typename TileRec<E, T>::Code code[E];
   alignas(16) T val[E];
-  T dinv;
+  struct alignas(16) Tail {
+    typename TileRec<E, T>::Code code[E];
+    T dinv;
+  } tail;
 };
 
 // the LDS word at a byte address (as kept in the packed records)
@@ -409,10 +424,15 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
         asm volatile("" : "+s"(at));
         const char *rec = pack + at;
         ld_pieces<R::kVal, R::kValPiece>(rec, lane, st[k].val);
-        ld_pieces<R::kCode, R::kCodePiece>(rec + R::kCodeAt, lane, st[k].code);
-        if constexpr (DIAG)
-          st[k].dinv = *reinterpret_cast<const T *>(rec + R::kDinvAt +
-                                                    static_cast<unsigned>(lane) * sizeof(T));
+        if constexpr (R::kJoined) {
+          static_assert(sizeof(st[k].tail) == R::kCodePiece, "addresses and 1/d in one load");
+          ld_pieces<R::kCodePiece, R::kCodePiece>(rec + R::kCodeAt, lane, &st[k].tail);
+        } else {
+          ld_pieces<R::kCode, R::kCodePiece>(rec + R::kCodeAt, lane, st[k].tail.code);
+          if constexpr (DIAG)
+            st[k].tail.dinv = *reinterpret_cast<const T *>(
+                rec + R::kDinvAt + static_cast<unsigned>(lane) * sizeof(T));
+        }
         at += R::kBytes;
       };
       // sched_barrier keeps the scheduler from reordering the groups' loads,
@@ -437,7 +457,7 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
       auto read_row = [&](const TileStage<E, T> &g, int bpos) {
         bv = bslot(bpos);
 #pragma unroll
-        for (int e = 0; e < E; ++e) xv[e] = *lds_at<V>(R::address(g.code[e]));
+        for (int e = 0; e < E; ++e) xv[e] = *lds_at<V>(R::address(g.tail.code[e]));
       };
       if (nblk > 0 && !tile_wait(&s_b[0], 0)) s_late = 1;
       lds_fence();
@@ -468,7 +488,7 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
           // lane's result is the one read and published)
           acc = group_sum<RL>(acc);
           A v = A(bv) - acc;
-          if constexpr (DIAG) v = v * A(tile_val(st[k].dinv));
+          if constexpr (DIAG) v = v * A(tile_val(st[k].tail.dinv));
           const V out = V(v);
           slot(base + k * kTileLanes) = out;
           code_order();
@@ -721,7 +741,7 @@ __global__ void k_tile_pack(int64_t slots, const int *__restrict__ src,
   }
   T d = T();
   if (dinv && dpos[t] >= 0) d = dinv[dpos[t]];
-  *reinterpret_cast<T *>(rec + R::kDinvAt + lane * sizeof(T)) = d;
+  *reinterpret_cast<T *>(rec + R::kDinvAt + lane * R::kDinvStep) = d;
 }
 
 template <int E, typename T>
@@ -739,10 +759,15 @@ void tile_pack(TrsvPlan &P, hipStream_t s) {
 
 // the packed records of one precision follow the level-ordered values
 void tile_pack(TrsvPlan &P, la_dtype dt, hipStream_t s) {
-  const bool e4 = P.t_maxe == 4;
-  if (dt == LA_F64) e4 ? tile_pack<4, double>(P, s) : tile_pack<kTileMaxEntries, double>(P, s);
-  else if (dt == LA_F32) e4 ? tile_pack<4, float>(P, s) : tile_pack<kTileMaxEntries, float>(P, s);
-  else e4 ? tile_pack<4, bf16>(P, s) : tile_pack<kTileMaxEntries, bf16>(P, s);
+  auto pack = [&](auto v) {
+    using T = decltype(v);
+    if (P.t_maxe == 2) tile_pack<2, T>(P, s);
+    else if (P.t_maxe == 4) tile_pack<4, T>(P, s);
+    else tile_pack<kTileMaxEntries, T>(P, s);
+  };
+  if (dt == LA_F64) pack(double());
+  else if (dt == LA_F32) pack(float());
+  else pack(bf16());
 }
 
 template <int E, int RL, int NB, int H, typename T, typename V, typename A, bool DIAG>
@@ -777,7 +802,8 @@ void launch_syncfree(TrsvPlan &P, const T *val, const T *diag, const V *b, V *x,
     // where a group takes longer (up to 18 values each). Measured per apply,
     // 4 x 1 / 4 x 2 / 2 x 4 (fetchers x groups): 512^2 428 / 400 / 393 us,
     // 56^3 27-point FP32 525 / 472 / 582 us
-    if (P.t_maxe == 4) tiled_launch<4, 1, 4, 2, T, V, A, DIAG>(P, b, x, s);
+    if (P.t_maxe == 2) tiled_launch<2, 1, 4, 2, T, V, A, DIAG>(P, b, x, s);
+    else if (P.t_maxe == 4) tiled_launch<4, 1, 4, 2, T, V, A, DIAG>(P, b, x, s);
     else if (P.t_rlanes == 1) tiled_launch<E8, 1, 4, 2, T, V, A, DIAG>(P, b, x, s);
     else tiled_launch<E8, RW, 2, 4, T, V, A, DIAG>(P, b, x, s);
     LA_HIP(hipGetLastError());

@@ -410,7 +410,7 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
   // source entry of each (row entries keep their stored order, the first
   // maxe on the row's first lane) and the halo fetch lists.
   out.rlanes = rl;
-  out.maxe = rl == 1 && maxe <= 4 ? 4 : kTileMaxEntries;
+  out.maxe = rl > 1 || maxe > 4 ? kTileMaxEntries : maxe > 2 ? 4 : 2;
   const int E = out.maxe;
   const int zero_slot = kTileWindow * lanes;
   std::vector<int> slot_of(static_cast<size_t>(n)), grp_of(static_cast<size_t>(n));

@@ -542,3 +542,41 @@ def test_tiled_solver_blocks_and_rings(dev, name, vec):
         bad[r] = np.nan
         refn = orc.backward_sub(o, D, bad) if upper else orc.forward_sub(o, bad)
         assert np.array_equal(nan.cpu().numpy(), np.isnan(refn))
+
+
+@pytest.mark.parametrize("shape", [(40, 34), (41, 33), (64, 64), (67, 131), (130, 33)])
+@pytest.mark.parametrize("val", [la.F64, la.F32, la.BF16])
+@pytest.mark.parametrize("vec", ["f64", "f32"])
+def test_tiled_two_entries_a_row(dev, shape, val, vec):
+    """Triangles with at most two entries a row (5-point operators) take
+    records of their own: whole and cut tiles, every value precision, unit and
+    stored diagonals. FP64 values and vectors against the oracle (1e-12). The
+    others against the level-by-level solve of the same plan: a row adds at
+    most 4 roundings of 2^-24 on either side to what its inputs carry, and the
+    factors' off-diagonal row sums stay below 0.98, so 2 * 4 * 2^-24 / 0.02 =
+    2.4e-5 bounds the relative difference; 1e-4 is allowed."""
+    import torch
+    A = la.gen.laplace3d(shape[0], shape[1], 1)
+    L, D, U = la.split_ldu(la.iluk(A, 0))
+    assert max(np.diff(L.ai).max(), np.diff(U.ai).max()) == 2
+    exact = val == la.F64 and vec == "f64"
+    dt = torch.float64 if vec == "f64" else torch.float32
+    b = la.gen.uniform(A.n, 23)
+    bt = torch.tensor(b, device=dev, dtype=dt)
+    for T, diag, upper in ((L, None, False), (U, D, True)):
+        S = la.TriangularSolve(T, diag, upper=upper)
+        assert S.info()["tiled"], shape
+        if val != la.F64:
+            S.add_dtype(val)
+        x = torch.zeros_like(bt)
+        S.solve(bt, x, val=val)
+        if exact:
+            o = orc.CSR(T.n, T.ai, T.aj, T.av)
+            ref = orc.backward_sub(o, D, b) if upper else orc.forward_sub(o, b)
+        else:
+            y = torch.zeros_like(bt)
+            S.solve(bt, y, mode=la.TRSV_LEVEL, val=val)
+            ref = y.cpu().numpy()
+        err = np.abs(x.cpu().numpy() - ref).max() / np.abs(ref).max()
+        print("case", shape, val, vec, "upper" if upper else "lower", "err", err, flush=True)
+        assert err <= (1e-12 if exact else 1e-4)
