@@ -338,24 +338,27 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
     return false;
   }
   const int rows_per_group = lanes / rl;
-  // rows of each tile by (level, index); tiles by their first level
-  std::vector<int> order(static_cast<size_t>(n));
-  for (int i = 0; i < n; ++i) order[i] = i;
+  // rows of each tile by (level, index), a tile's rows sorted by themselves (one
+  // sort over all rows took a quarter of the plan: 100x96x90 ILU(0) preconditioner
+  // 360 -> 257 ms, 512^2 90 -> 55 ms); tiles by their first level
   // (rows that other tiles read come first in their level, by the reading
   // tile: the solve hands those over as one contiguous run per group)
   std::vector<int> reader(static_cast<size_t>(n), INT32_MAX);
   for (int i = 0; i < n; ++i)
     for (int q = ai[i]; q < ai[i + 1]; ++q)
       if (part[aj[q]] != part[i]) reader[aj[q]] = std::min(reader[aj[q]], part[i]);
-  std::sort(order.begin(), order.end(), [&](int a, int b) {
-    if (part[a] != part[b]) return part[a] < part[b];
-    if (level[a] != level[b]) return level[a] < level[b];
-    if (reader[a] != reader[b]) return reader[a] < reader[b];
-    return a < b;
-  });
-  std::vector<int> pstart(static_cast<size_t>(nparts) + 1, 0);
+  std::vector<int> pstart(static_cast<size_t>(nparts) + 1, 0), order(static_cast<size_t>(n));
   for (int i = 0; i < n; ++i) pstart[part[i] + 1]++;
   for (int p = 0; p < nparts; ++p) pstart[p + 1] += pstart[p];
+  std::vector<int> put(pstart.begin(), pstart.end() - 1);
+  for (int i = 0; i < n; ++i) order[put[part[i]]++] = i;
+#pragma omp parallel for schedule(dynamic, 1)
+  for (int p = 0; p < nparts; ++p)
+    std::sort(order.begin() + pstart[p], order.begin() + pstart[p + 1], [&](int a, int b) {
+      if (level[a] != level[b]) return level[a] < level[b];
+      if (reader[a] != reader[b]) return reader[a] < reader[b];
+      return a < b;
+    });
   std::vector<int> porder(static_cast<size_t>(nparts));
   for (int p = 0; p < nparts; ++p) porder[p] = p;
   if (box) {
