@@ -283,7 +283,7 @@ __device__ __forceinline__ void lds_store(int *p, int v) {
 // piece for all 64 lanes, so that every load covers one contiguous run. Issuing
 // the loads is a quarter of the solving wavefront's time (128^2, FP64: 273
 // cycles a group, 200-210 without them; the LDS write, read and four
-// multiply-adds take the rest), so with two values per lane 1/d sits in the
+// multiply-adds take the rest), so with two FP64 values per lane 1/d sits in the
 // addresses' piece: two loads a group instead of four (5-point IC(0) per
 // apply, FP64: 128^2 94.4 -> 84.8 us, 512^2 338 -> 303 us). An
 // address is a byte address in 32 bits, ready to use; with eight values per
@@ -301,9 +301,9 @@ struct TileRec {
   static constexpr int kVal = E * static_cast<int>(sizeof(T));
   static constexpr int kValPiece = kVal < 16 ? kVal : 16;
   static constexpr int kCode = E * static_cast<int>(sizeof(Code));
-  static constexpr int kCodePiece = 16;
+  static constexpr bool kJoined = E == 2 && sizeof(T) == 8;  // 1/d behind the addresses
+  static constexpr int kCodePiece = kJoined || kCode > 16 ? 16 : kCode;
   static constexpr int kCodeAt = kTileLanes * kVal;
-  static constexpr bool kJoined = E == 2;  // 1/d behind the addresses
   static constexpr int kDinvAt = kCodeAt + (kJoined ? kCode : kTileLanes * kCode);
   static constexpr int kDinvStep = kJoined ? kCodePiece : static_cast<int>(sizeof(T));
   static constexpr int kBytes =
@@ -424,9 +424,14 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
         asm volatile("" : "+s"(at));
         const char *rec = pack + at;
         ld_pieces<R::kVal, R::kValPiece>(rec, lane, st[k].val);
-        if constexpr (R::kJoined) {
+        // (a load's registers must all be used: the compiler puts other values
+        // into those that are not, and then waits for the load at once)
+        if constexpr (R::kJoined && DIAG) {
           static_assert(sizeof(st[k].tail) == R::kCodePiece, "addresses and 1/d in one load");
           ld_pieces<R::kCodePiece, R::kCodePiece>(rec + R::kCodeAt, lane, &st[k].tail);
+        } else if constexpr (R::kJoined) {
+          *reinterpret_cast<tile_u2 *>(st[k].tail.code) = __builtin_nontemporal_load(
+              reinterpret_cast<const tile_u2 *>(rec + R::kCodeAt + lane * 16u));
         } else {
           ld_pieces<R::kCode, R::kCodePiece>(rec + R::kCodeAt, lane, st[k].tail.code);
           if constexpr (DIAG)
