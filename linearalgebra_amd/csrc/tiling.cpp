@@ -154,14 +154,22 @@ double correlation(const std::vector<int> &a, const std::vector<int> &b) {
 // The tile edge: the smallest power of two whose tile count fits the resident
 // workgroups, then doubled while a tile's rows of one level still fit one
 // group (the solve takes as long over a group of 64 rows as over one of 8, and
-// every tile on the way costs a hand-over), at least kMinTiles tiles remain
-// and a tile's faces stay small (kMaxFace rows of other tiles). Measured per
+// every tile on the way costs a hand-over), at least kMinTiles tiles remain,
+// a tile's faces stay small (kMaxFace entries in other tiles) and nothing
+// that the layout is refused for appears: a larger tile takes in dependencies
+// that crossed tiles before, and in some row orders (rows back and forth,
+// dissected, blocks by colour) they reach beyond the LDS window. (A layout
+// refused for that leaves the solve to the level-chunk schedule: 512^2 in
+// 32 x 32 blocks by colour, FP64, lower triangle 191 us against 37 us with
+// tiles, 128^2 with rows back and forth 5.4 against 2.7 ms.) Measured per
 // apply, smallest edge -> this rule: 128^2 5-point IC(0) FP64 (256 -> 4 tiles)
 // 171 -> 122 us, 512^2 (256 -> 64 tiles) 372 -> 364 us.
 constexpr int kMinTiles = 4;
 constexpr int kMaxFace = 8192;
+constexpr double kMaxRemote = 0.35;  // entries that cross tiles
 bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes, int max_parts,
-               int max_rows, std::vector<int> &part, int &tau, int &nparts, std::string &why) {
+               int max_rows, int max_halo, std::vector<int> &part, int &tau, int &nparts,
+               std::string &why) {
   const int64_t nnz = ai[n];
   // symmetric adjacency of the triangle (T + T^T)
   std::vector<int> ptr(static_cast<size_t>(n) + 1, 0), adj(static_cast<size_t>(2 * nnz));
@@ -230,7 +238,9 @@ bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes,
   auto tile_of = [&](int i, int t, int nv) {
     return static_cast<size_t>(u[i] / t) * nv + v[i] / t;
   };
-  std::vector<int> by_level;  // rows level by level, when a larger edge is tried
+  // rows level by level and their groups in their tiles, when a larger edge
+  // is tried
+  std::vector<int> by_level, group;
   for (int t = 2; t <= 4096; t *= 2) {
     const int nu = umax / t + 1, nv = vmax / t + 1;
     if (static_cast<int64_t>(nu) * nv > 4 * static_cast<int64_t>(max_parts)) continue;
@@ -246,7 +256,9 @@ bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes,
       continue;
     }
     if (tau) {
-      // a larger edge: one group per level, tiles and faces as above
+      // a larger edge: one group per level, tiles and faces as above (the
+      // layout's own limits on the window, the halo and the entries that cross
+      // tiles are then kept, too)
       if (used < kMinTiles) break;
       if (by_level.empty()) {
         int top = 0;
@@ -256,8 +268,12 @@ bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes,
         for (int l = 0; l <= top; ++l) at[l + 1] += at[l];
         by_level.resize(static_cast<size_t>(n));
         for (int i = 0; i < n; ++i) by_level[at[level[i]]++] = i;
+        group.resize(static_cast<size_t>(n));
       }
-      std::vector<int> seen(cnt.size(), -1), rows(cnt.size(), 0), face(cnt.size(), 0);
+      std::vector<int> seen(cnt.size(), -1), rows(cnt.size(), 0), face(cnt.size(), 0),
+          groups(cnt.size(), 0);
+      const int most = std::min(kMaxFace, max_halo);
+      int64_t cross = 0;
       bool fits = true;
       for (int k = 0; k < n && fits; ++k) {
         const int i = by_level[k];
@@ -265,12 +281,19 @@ bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes,
         if (seen[c] != level[i]) {
           seen[c] = level[i];
           rows[c] = 0;
+          groups[c]++;
         }
+        group[i] = groups[c];
         fits = ++rows[c] <= lanes;
-        for (int q = ai[i]; q < ai[i + 1]; ++q) face[c] += tile_of(aj[q], t, nv) != c;
-        fits = fits && face[c] <= kMaxFace;
+        for (int q = ai[i]; q < ai[i + 1]; ++q) {
+          const bool other = tile_of(aj[q], t, nv) != c;
+          face[c] += other;
+          cross += other;
+          fits = fits && (other || group[i] - group[aj[q]] < kTileWindow);
+        }
+        fits = fits && face[c] <= most;
       }
-      if (!fits) break;
+      if (!fits || cross > kMaxRemote * nnz) break;
     }
     std::vector<int> id(cnt.size(), -1);
     nparts = 0;
@@ -303,7 +326,8 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
   int tau = 0, nparts = 0, rl = 1;
   bool box = false;
   if (maxe <= kTileMaxEntries) {
-    if (!bfs_tiles(n, ai, aj, level, lanes, max_parts, max_rows, part, tau, nparts, why))
+    if (!bfs_tiles(n, ai, aj, level, lanes, max_parts, max_rows, max_halo, part, tau, nparts,
+                   why))
       return false;
   } else if (maxe <= kTileRowLanes * kTileMaxEntries) {
     int nx = 0, ny = 0, nz = 0;
@@ -482,7 +506,7 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
   }
   // (box tiles are narrow: most of their reads cross tiles, but each
   // value is fetched once and the halo is bounded above)
-  if (!box && out.remote_frac > 0.35) {
+  if (!box && out.remote_frac > kMaxRemote) {
     why = "too many values cross tiles";
     return false;
   }

@@ -233,3 +233,136 @@ def test_tile_edge_rule(tl, dims, most):
         tl.tiling_sizes(_p(v))
         lv = _levels(T.n, np.asarray(T.ai), np.asarray(T.aj), upper)
         assert v[1] <= nparts * (lv.max() + 1)  # one group per level and tile
+
+
+def _serpentine(nx, ny):
+    c = np.arange(nx * ny)
+    x, y = c % nx, c // nx
+    return y * nx + np.where(y % 2 == 1, nx - 1 - x, x)
+
+
+def _dissected(nx, ny, leaf):
+    """Nested dissection: halves along the longer side, then the line that
+    parts them; blocks of at most leaf x leaf nodes by rows."""
+    key, at = np.zeros(nx * ny, np.int64), 0
+
+    def rec(x0, x1, y0, y1):
+        nonlocal at
+        if x0 >= x1 or y0 >= y1:
+            return
+        if max(x1 - x0, y1 - y0) <= leaf:
+            xs, ys = np.arange(x0, x1), np.arange(y0, y1)
+        elif x1 - x0 >= y1 - y0:
+            m = (x0 + x1) // 2
+            rec(x0, m, y0, y1)
+            rec(m + 1, x1, y0, y1)
+            xs, ys = np.array([m]), np.arange(y0, y1)
+        else:
+            m = (y0 + y1) // 2
+            rec(x0, x1, y0, m)
+            rec(x0, x1, m + 1, y1)
+            xs, ys = np.arange(x0, x1), np.array([m])
+        ids = (ys[:, None] * nx + xs[None, :]).ravel()
+        key[ids] = at + np.arange(len(ids))
+        at += len(ids)
+
+    rec(0, nx, 0, ny)
+    return key
+
+
+def _two_colours(nx, ny, s):
+    """Blocks of s x s nodes, all blocks of one colour before the other's."""
+    c = np.arange(nx * ny)
+    x, y = c % nx, c // nx
+    block = ((x // s + y // s) % 2 * ny + y // s) * nx + x // s
+    return (block * s + y % s) * s + x % s
+
+
+def _halves(nx, ny):
+    """One-level dissection: the two halves, then the column between them."""
+    c = np.arange(nx * ny)
+    return np.where(c % nx < nx // 2, 0, np.where(c % nx > nx // 2, 1, 2)) * len(c) + c
+
+
+def _ordered_triangle(dims, key, upper, seed):
+    """A triangle of the 5-point (7-point) pattern, rows in the order of key."""
+    import scipy.sparse as sp
+    A = la.gen.poisson2d(*dims) if len(dims) == 2 else la.gen.laplace3d(*dims)
+    M = sp.csr_matrix((A.av, A.aj, A.ai), shape=(A.n, A.n))
+    if key is not None:
+        p = np.argsort(key, kind="stable")
+        M = M[p][:, p]
+    T = (sp.triu(M, 1) if upper else sp.tril(M, -1)).tocsr()
+    T.sort_indices()
+    T.data = np.random.default_rng(seed).uniform(-1, 1, T.nnz) / 8
+    return orc.CSR(A.n, T.indptr, T.indices, T.data)
+
+
+def _replay_resident(tl, T, diag, b, upper):
+    """As _replay, for tiles that read each other: every tile is resident (at
+    most one per compute unit) and goes on whenever the values its next group
+    reads from other tiles are solved."""
+    ok, why, ai, aj = _build(tl, T, upper)
+    assert ok, why
+    v = np.zeros(7, np.int32)
+    tl.tiling_sizes(_p(v))
+    nparts, ngroups, rl, E, hmax, nrf, ncode = (int(t) for t in v)
+    pg, gr, tp = (np.zeros(k, np.int32) for k in (nparts + 1, ngroups + 1, T.n))
+    tc, ts = np.zeros(ncode, np.int32), np.zeros(ncode, np.int32)
+    rp = np.zeros(ngroups + 1, np.int32)
+    rc, rs = np.zeros(max(nrf, 1), np.int32), np.zeros(max(nrf, 1), np.int32)
+    tl.tiling_get(_p(pg), _p(gr), _p(tp), _p(tc), _p(ts), _p(rp), _p(rc), _p(rs))
+    tc, ts = tc.reshape(T.n, rl * E), ts.reshape(T.n, rl * E)
+    av = np.append(np.asarray(T.av, np.float64), 0.0)  # (-1: padding)
+    x = np.full(T.n, np.nan)
+    # per tile the window, the zero slot, and the halo from the back
+    lds = np.full((nparts, ZERO_SLOT + 1 + max(hmax, 1)), np.nan)
+    lds[:, ZERO_SLOT] = 0.0
+    at = pg[:-1].copy()
+    moved = True
+    while moved:
+        moved = False
+        for p in range(nparts):
+            while at[p] < pg[p + 1]:
+                g = at[p]
+                q = slice(rp[g], rp[g + 1])
+                if np.isnan(x[rc[q]]).any():
+                    break
+                lds[p, -1 - rs[q]] = x[rc[q]]
+                rows = np.arange(gr[g], gr[g + 1])
+                val = lds[p, tc[rows]]
+                assert not np.isnan(val).any(), ("read before written", p, g)
+                out = (b[tp[rows]] - (av[ts[rows]] * val).sum(1)) / diag[tp[rows]]
+                base = (g - pg[p]) % WINDOW * LANES
+                for w in range(rl):
+                    lds[p, base + rl * (rows - gr[g]) + w] = out
+                x[tp[rows]] = out
+                at[p] += 1
+                moved = True
+    assert (at == pg[1:]).all(), "tiles wait for each other"
+    return x, nparts, rl
+
+
+@pytest.mark.parametrize("dims,order", [
+    ((48, 48), "serpentine"), ((60, 200), "serpentine"), ((128, 128), "serpentine"),
+    ((40, 40), "dissected"), ((56, 56), "dissected"), ((64, 64), "dissected"),
+    ((128, 128), "two colours of 32"), ((128, 128), "two colours of 16"), ((128, 128), "halves")])
+@pytest.mark.parametrize("upper", [False, True])
+def test_tile_edge_keeps_the_window(tl, dims, order, upper):
+    """Row orders in which a larger tile's own dependencies would reach
+    beyond the LDS window: the tiles stay at an edge whose layout is
+    accepted, and it replays to plain substitution."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as spl
+    key = {"serpentine": lambda: _serpentine(*dims), "dissected": lambda: _dissected(*dims, 4),
+           "two colours of 32": lambda: _two_colours(*dims, 32),
+           "two colours of 16": lambda: _two_colours(*dims, 16),
+           "halves": lambda: _halves(*dims)}[order]()
+    T = _ordered_triangle(dims, key, upper, 3)
+    D = 1.0 + np.random.default_rng(4).random(T.n)
+    b = la.gen.uniform(T.n, 24)
+    x, nparts, rl = _replay_resident(tl, T, D, b, upper)
+    M = sp.csr_matrix((T.av, T.aj, T.ai), shape=(T.n, T.n)) + sp.diags(D)
+    ref = spl.spsolve_triangular(M.tocsr(), b, lower=not upper)
+    assert 4 <= nparts <= 256 and rl == 1
+    assert np.abs(x - ref).max() <= 1e-12 * np.abs(ref).max()
