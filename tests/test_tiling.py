@@ -366,3 +366,22 @@ def test_tile_edge_keeps_the_window(tl, dims, order, upper):
     ref = spl.spsolve_triangular(M.tocsr(), b, lower=not upper)
     assert 4 <= nparts <= 256 and rl == 1
     assert np.abs(x - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("dims,order,tiles", [
+    ((128, 128), None, 4),         # smallest edge 8; 64 is the last with 64 rows a level
+    ((512, 512), None, 64),        # edge 128: 128 rows a level in 16 tiles
+    ((60, 60), None, 4),           # edge 64: one tile
+    ((16, 16, 500), None, 4),      # edge 8: faces of 2 x 8 x 500 entries
+    ((16, 16, 520), None, 16),     # edge 8: 2 x 8 x 520 entries, past 8192
+    ((60, 200), "serpentine", 200),  # edge 8: past the window
+    ((128, 128), "two colours of 16", 64)])
+def test_tile_edge_chosen(tl, dims, order, tiles):
+    """Where the growth of the tile edge ends, for each of its reasons."""
+    key = {None: lambda: None, "serpentine": lambda: _serpentine(*dims),
+           "two colours of 16": lambda: _two_colours(*dims, 16)}[order]()
+    ok, why, _, _ = _build(tl, _ordered_triangle(dims, key, False, 5), False)
+    assert ok, why
+    v = np.zeros(7, np.int32)
+    tl.tiling_sizes(_p(v))
+    assert v[0] == tiles
