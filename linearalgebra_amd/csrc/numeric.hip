@@ -263,12 +263,6 @@ __global__ __launch_bounds__(64) void k_ic_rows(int k0, const int *__restrict__ 
 // IC(0) (255 levels) 1.18 -> 0.36 ms (with the refreshed solve plans).
 constexpr int kFacWaves = 4;
 constexpr int kFacMaxLanes = 64;
-// workgroups: this many levels of chunks at a time (clamped to 64 .. 1024),
-// so that the pattern work of later rows is done while they wait. 27-point
-// ILU(1) on 48^3 with 1 / 2 / 4 / 8 / 16 levels ahead (8 wavefronts): 8.3 /
-// 6.1 / 3.4 / 2.3 / 2.2 ms; 72^3 IC(0) with 4 / 8 / 32: 490 / 465 / 573 us
-// (more pollers)
-constexpr int kFacAhead = 12;
 constexpr uint64_t kFacWaitTicks = 20000000;  // 0.2 s of the 100 MHz clock
 
 template <int G>
@@ -716,8 +710,7 @@ void factor_rows(NumericPlan &N, const double *a_vals, hipStream_t s) {
   hipLaunchKernelGGL(k_factor_mark, dim3(2048), dim3(256), 0, s, N.nnzF, fav);
   LA_HIP(hipGetLastError());
   const int levels = std::max<int>(1, static_cast<int>(N.level_ptr.size()) - 1);
-  const unsigned grid = static_cast<unsigned>(
-      std::min(N.nchunks, std::clamp(kFacAhead * N.nchunks / levels, 64, 1024)));
+  const unsigned grid = static_cast<unsigned>(factor_workgroups(N.nchunks, levels));
   const bool add = N.ic && N.additive;
 #define LA_FAC(G, IC)                                                                          \
   hipLaunchKernelGGL((k_factor_rows<G, IC>), dim3(grid), dim3(64 * kFacWaves), 0, s, N.nchunks, \
