@@ -86,8 +86,24 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
                        int max_parts, int max_rows, int max_halo, TileLayout &out,
                        std::string &why);
 
-// Sync-free device factorisation (numeric.hip).
-// Workgroups: kFacAhead levels of chunks at a time (clamped to 64 .. 1024),
+// Device factorisation (numeric.hip).
+// One sync-free launch, or one launch per level? The first gives every row as
+// many lanes as the longest one needs and keeps about 4096 wavefronts in
+// flight, 0.049 ns per row and lane, and a level costs it 1.4-4 us; the second
+// pays about 14 us a level and 0.25 ns a row with 0.28 ns an elimination. So
+// levels decide, except where few of them hold very many rows that are much
+// shorter than the longest. One launch / one per level, ILU(0) of a random
+// graph with n rows of mean degree d: n = 500K, d = 4 (17 levels, 32 lanes)
+// 821 / 675 us, d = 8 (26 levels, 32 lanes) 857 / 1164 us; n = 2M, d = 2 (12
+// levels, 16 lanes) 1.58 / 1.21 ms, d = 4 (32 lanes) 3.06 / 1.87 ms. 128^3
+// 7-point cells by colour (2 levels, 8 lanes) 0.91 / 2.00 ms; 1M rows of a
+// diagonal and one of 60 entries (64 lanes) 2.93 / 0.35 ms.
+inline bool factor_one_launch(int64_t rows, int64_t levels, int lanes, int64_t eliminations) {
+  const double one = 4000.0 * levels + 0.049 * rows * lanes;
+  const double per_level = 14000.0 * levels + 0.25 * rows + 0.28 * eliminations;
+  return one <= per_level;
+}
+// Workgroups of the one launch: kFacAhead levels of chunks at a time (clamped to 64 .. 1024),
 // so that the pattern work of later rows is done while they wait. 27-point
 // ILU(1) on 48^3 with 1 / 2 / 4 / 8 / 16 levels ahead (8 wavefronts): 8.3 /
 // 6.1 / 3.4 / 2.3 / 2.2 ms; 72^3 IC(0) with 4 / 8 / 32: 490 / 465 / 573 us

@@ -22,8 +22,8 @@
 // as in the reference's x86-64 build.
 //
 // Rows of at most 64 entries (and eliminations): one launch, sync-free
-// (k_factor_rows). Longer rows: level by level (one launch per level of the
-// factorisation's dependency DAG, which is the lower triangular solve's), one
+// (k_factor_rows). Longer rows, and few levels of very many rows (see
+// factor_one_launch): level by level (one launch per level of the factorisation's dependency DAG, which is the lower triangular solve's), one
 // 64-lane workgroup per row with the row's columns and values in LDS; for
 // each eliminating row k the lanes take k's entries, find their column in the
 // row by binary search and update it. A row longer than kRowCap is done by
@@ -513,15 +513,20 @@ void finish_plans(Prec &P, NumericPlan &N, const std::vector<int> &Li, const std
   P.tmp[1].alloc(sizeof(float) * std::max(n, 1));
   LA_HIP(hipStreamSynchronize(s));
 }
-// The sync-free form applies when a row and its eliminations fit a wavefront:
-// the fewest lanes per row that hold both (at least 4).
+// The sync-free form applies when a row and its eliminations fit a wavefront
+// and it is the faster one: the fewest lanes per row that hold both (at least
+// 4).
 void plan_sync_free(NumericPlan &N, const std::vector<int> &fai, const std::vector<int64_t> &a2f,
-                    int max_elim, const std::vector<int> &dpos, hipStream_t s) {
+                    int max_elim, int64_t eliminations, const std::vector<int> &dpos,
+                    hipStream_t s) {
   int longest = max_elim;
   for (int i = 0; i < N.n; ++i) longest = std::max(longest, fai[i + 1] - fai[i]);
   if (longest > kFacMaxLanes || N.nnzA >= INT32_MAX) return;
-  N.lanes = 4;
-  while (N.lanes < longest) N.lanes *= 2;
+  int lanes = 4;
+  while (lanes < longest) lanes *= 2;
+  const int levels = std::max<int>(1, static_cast<int>(N.level_ptr.size()) - 1);
+  if (!factor_one_launch(N.n, levels, lanes, eliminations)) return;
+  N.lanes = lanes;
   std::vector<int> f2a(static_cast<size_t>(N.nnzF), -1), chunks;
   for (size_t a = 0; a < a2f.size(); ++a)
     if (a2f[a] >= 0) f2a[a2f[a]] = static_cast<int>(a);
@@ -576,7 +581,8 @@ std::unique_ptr<Prec> make_prec_ilu_gpu(int n, int base, const int *ai, const in
   upload_vec(N.a2f, a2f, s);
   N.diag.alloc(sizeof(double) * std::max(n, 1));
   finish_plans(*P, N, Li, Lj, Ls, nullptr, Ui, Uj, Us, dpos, s);
-  plan_sync_free(N, fai, a2f, 0, std::vector<int>(dpos.begin(), dpos.end()), s);
+  plan_sync_free(N, fai, a2f, 0, static_cast<int64_t>(Lj.size()),
+                 std::vector<int>(dpos.begin(), dpos.end()), s);
   N.h_fai = std::move(fai);
   N.h_faj = std::move(faj);
   return P;
@@ -697,7 +703,7 @@ std::unique_ptr<Prec> make_prec_ic_gpu(int n, int base, const int *ai, const int
   finish_plans(*P, N, Li, Lj, Ls, &dsrc, Ui, Uj, Us, dsrc, s);
   int max_elim = 0;
   for (int j = 0; j < n; ++j) max_elim = std::max(max_elim, pptr[j + 1] - pptr[j]);
-  plan_sync_free(N, fai, a2f, max_elim, {}, s);
+  plan_sync_free(N, fai, a2f, max_elim, static_cast<int64_t>(pk.size()), {}, s);
   N.h_fai = std::move(fai);
   N.h_faj = std::move(faj);
   return P;

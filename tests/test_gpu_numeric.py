@@ -246,3 +246,31 @@ def test_banded_factor_bitwise_host(dev, width, kind):
             P.refactor(torch.tensor(bad, device=dev))
         P.refactor(torch.tensor(A.av, device=dev))
         assert np.array_equal(P.factor().av, F.av)
+
+
+@pytest.mark.parametrize("n", [2000, 20000])
+@pytest.mark.parametrize("kind", ["ilu", "ic"])
+def test_one_long_row_bitwise_host(dev, n, kind):
+    """A diagonal and one row of 60 entries: one launch (2000 rows) and one
+    launch per level (20000 rows, where 64 lanes a row cost more than the two
+    launches), bitwise the host's factor."""
+    import torch
+    rng = np.random.default_rng(n)
+    at = np.sort(rng.choice(n - 1, 59, replace=False))
+    v = rng.uniform(-1, 0, 59)
+    last = np.full(59, n - 1)
+    rows = np.concatenate([np.arange(n), last, at])
+    cols = np.concatenate([np.arange(n), at, last])
+    vals = np.concatenate([np.full(n, 64.0), v, v])
+    o = np.lexsort((cols, rows))
+    ai = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))])
+    A = la.CSR(n, ai, cols[o], vals[o])
+    if kind == "ilu":
+        F, P = la.iluk(A, 0), la.Preconditioner.ilu_gpu(A, 0)
+    else:
+        (F, ok), P = la.icc(la.split_triangle(A, True), 0), la.Preconditioner.ic_gpu(A, 0)
+    for _ in range(2):
+        P.refactor(torch.tensor(A.av, device=dev))
+        G = P.factor()
+        assert np.array_equal(G.ai, F.ai) and np.array_equal(G.aj, F.aj)
+        assert np.array_equal(G.av, F.av)
