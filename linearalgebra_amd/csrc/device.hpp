@@ -141,6 +141,8 @@ struct TrsvPlan {
   // the values tiles read from each other: t_mstride slots per group, its
   // shared rows first (FP64 or FP32, as the solve's vectors)
   DevBuf t_mail;
+  // b in the order of the records, where the halo leaves LDS no room for it
+  DevBuf t_stage;
   int t_mstride = 0;
   int64_t t_nmail = 0;
   unsigned t_wgs = 0;   // workgroups launched

@@ -250,7 +250,9 @@ __global__ __launch_bounds__(NT) void k_trsv_syncfree(
 constexpr int kTileLanes = 64;
 constexpr int kTileDepth = 8;  // groups whose rows sit in registers; one block of the I/O wavefronts
 constexpr int kTileIo = 2;     // I/O wavefronts
-constexpr int kTileCtl = 64;   // bytes of LDS control words, ahead of the slots
+// bytes of LDS control words, ahead of the slots (a cache line, or what they
+// need where b is staged)
+constexpr int tile_ctl(bool staged) { return staged ? 40 : 64; }
 // Groups of padding the packed rows end with (the solver runs up to
 // kTileDepth - 1 groups past a tile's last one and loads kTileDepth ahead),
 // and mail slots' spare groups per tile for the same reason.
@@ -344,13 +346,14 @@ template <> __device__ __forceinline__ float tile_val<bf16>(bf16 v) {
 __device__ __forceinline__ double tile_val(double v) { return v; }
 
 // one pipeline stage: a group's record for this lane
-template <int E, typename T>
+template <int E, typename T, typename V>
 struct TileStage {
   alignas(16) T val[E];
   struct alignas(16) Tail {
     typename TileRec<E, T>::Code code[E];
     T dinv;
   } tail;
+  V b;  // (only where b is staged)
 };
 
 // the LDS word at a byte address (as kept in the packed records)
@@ -373,27 +376,36 @@ __device__ __forceinline__ bool tile_wait(const int *p, int have) {
   return true;
 }
 
-template <int E, int RL, int NB, int H, typename T, typename V, typename A, bool DIAG>
+// STAGED: the halo (18424 to 19450 values) leaves no room for a ring of b. b
+// then holds the right-hand side in the order of the records (64 slots per
+// group, k_tile_stage), which the solver loads along with them: a launch and a
+// pass over b more, but the tiles stay. 27-point ILU(1) on 2304 x 6 x 6, lower
+// triangle, FP64 / FP32: 464 / 360 us, level chunks 1096 / 977 us (2302 x 6 x 6
+// with the ring 452 / 373 us); 7-point on 8 x 8 x 4700 715 / 538 us, level
+// chunks 1707 / 1625 us.
+template <int E, int RL, int NB, int H, typename T, typename V, typename A, bool DIAG,
+          bool STAGED>
 __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
     int nparts, const int *__restrict__ gptr, const int2 *__restrict__ rows,
     const char *__restrict__ pack, const int2 *__restrict__ reads, int rstride,
     const V *__restrict__ b, V *__restrict__ x, V *mail, int mstride, int ring, int hmax,
     int touch, unsigned *ctl, int *err) {
-  constexpr int D = kTileDepth;
+  constexpr int D = kTileDepth, kCtl = tile_ctl(STAGED);
   static_assert(D % (NB * H) == 0, "a group's fetcher is fixed by its place in the loop");
   static_assert(kTileIo <= kTileWindow / D, "a block's rows are listed before its results go out");
   using R = TileRec<E, T>;
   // LDS, all of it dynamic so that it starts at address 0 (a record's
   // addresses are then used as they are): control words, then 8-byte slots:
   // results of `ring` groups, the zero slot, the halo, b of `ring` groups
+  // (not if staged)
   extern __shared__ __align__(16) unsigned char smem[];
   int *const s_prog = reinterpret_cast<int *>(smem), *const s_b = s_prog + H;
   int &s_part = s_b[kTileIo], &s_late = s_b[kTileIo + 1], &s_done = s_b[kTileIo + 2];
-  static_assert((H + kTileIo + 3) * 4 <= kTileCtl, "control words");
+  static_assert((H + kTileIo + 3) * 4 <= kCtl, "control words");
   const int wave = static_cast<int>(threadIdx.x) / kTileLanes;
   const int lane = static_cast<int>(threadIdx.x) % kTileLanes;
-  unsigned char *const bring = smem + kTileCtl + 8 * (ring * kTileLanes + 1 + hmax);
-  auto slot = [&](int q) -> V & { return *reinterpret_cast<V *>(smem + kTileCtl + 8 * q); };
+  unsigned char *const bring = smem + kCtl + 8 * (ring * kTileLanes + 1 + hmax);
+  auto slot = [&](int q) -> V & { return *reinterpret_cast<V *>(smem + kCtl + 8 * q); };
   auto bslot = [&](int q) -> V & { return *reinterpret_cast<V *>(bring + 8 * q); };
   // The next tile's ticket and cleared control words, between two barriers.
   // The loop below must stay one loop of whole wavefronts: thread 0's work on
@@ -416,8 +428,9 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
     const int nblk = (ng + D - 1) / D;
     if (wave == 0) {
       __builtin_amdgcn_s_setprio(3);  // issue priority over the other wavefronts
-      TileStage<E, T> st[D];
+      TileStage<E, T, V> st[D];
       int64_t at = static_cast<int64_t>(g0) * R::kBytes;
+      const V *bat = b + static_cast<int64_t>(g0) * kTileLanes;
       auto load_rows = [&](int k) {  // the next group's record
         // (the offset is kept in scalar registers: scalar additions instead
         // of 64-bit vector address arithmetic per load)
@@ -439,6 +452,10 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
                 rec + R::kDinvAt + static_cast<unsigned>(lane) * sizeof(T));
         }
         at += R::kBytes;
+        if constexpr (STAGED) {
+          st[k].b = __builtin_nontemporal_load(bat + lane);
+          bat += kTileLanes;
+        }
       };
       // sched_barrier keeps the scheduler from reordering the groups' loads,
       // so that the loads in flight when the loop starts are as old as in
@@ -459,8 +476,9 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
       // in the rare other case. Hand-over and loads are issued while those
       // reads are on their way.
       V bv, xv[E];
-      auto read_row = [&](const TileStage<E, T> &g, int bpos) {
-        bv = bslot(bpos);
+      auto read_row = [&](const TileStage<E, T, V> &g, int bpos) {
+        if constexpr (STAGED) bv = g.b;
+        else bv = bslot(bpos);
 #pragma unroll
         for (int e = 0; e < E; ++e) xv[e] = *lds_at<V>(R::address(g.tail.code[e]));
       };
@@ -601,6 +619,7 @@ __global__ __launch_bounds__(kTileLanes * (1 + H + kTileIo)) void k_trsv_tiled(
         for (int u = 0; u < NI; ++u) to[u] = rp[(m * NI + u) * kTileLanes];
       };
       auto gather = [&] {
+        if constexpr (STAGED) return;
 #pragma unroll
         for (int u = 0; u < NI; ++u) {
           rb[u] = rid[u];
@@ -717,9 +736,19 @@ __global__ void k_tile_prep(int64_t n, V *mail, unsigned *ctl) {
   if (blockIdx.x == 0 && threadIdx.x < 16) ctl[threadIdx.x] = 0;
 }
 
-// 8-byte LDS slots: results and b of `ring` groups, the zero slot, the halo
-inline size_t tile_lds_bytes(int ring, int h_max) {
-  return kTileCtl + 8 * (2 * static_cast<size_t>(ring) * kTileLanes + 1 + h_max);
+// b in the order of the records: slot t's row (dpos: its level position, -1:
+// padding; perm: that position's row)
+template <typename V>
+__global__ void k_tile_stage(int64_t slots, const int *__restrict__ dpos,
+                             const int *__restrict__ perm, const V *__restrict__ b, V *out) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * kB + threadIdx.x;
+  if (t < slots) out[t] = dpos[t] >= 0 ? b[perm[dpos[t]]] : V(0);
+}
+
+// 8-byte LDS slots: results and, unless staged, b of `ring` groups, the zero
+// slot, the halo
+inline size_t tile_lds_bytes(int ring, int h_max, bool staged) {
+  return tile_ctl(staged) + 8 * ((staged ? 1 : 2) * static_cast<size_t>(ring) * kTileLanes + 1 + h_max);
 }
 
 // The packed records: slot t's entries from the level-ordered values
@@ -775,10 +804,22 @@ void tile_pack(TrsvPlan &P, la_dtype dt, hipStream_t s) {
   else pack(bf16());
 }
 
-template <int E, int RL, int NB, int H, typename T, typename V, typename A, bool DIAG>
+template <int E, int RL, int NB, int H, typename T, typename V, typename A, bool DIAG,
+          bool STAGED = false>
 void tiled_launch(TrsvPlan &P, const V *b, V *x, hipStream_t s) {
-  auto kern = k_trsv_tiled<E, RL, NB, H, T, V, A, DIAG>;
-  const size_t lds = tile_lds_bytes(P.t_ring, P.t_hmax);
+  if constexpr (!STAGED) {
+    if (P.t_stage.p) {
+      const int64_t slots = (static_cast<int64_t>(P.t_ngroups) + kTilePad) * kTileLanes;
+      hipLaunchKernelGGL(k_tile_stage<V>, dim3(static_cast<unsigned>((slots + kB - 1) / kB)),
+                         dim3(kB), 0, s, slots, P.t_dpos.as<int>(), P.perm.as<int>(), b,
+                         P.t_stage.as<V>());
+      LA_HIP(hipGetLastError());
+      tiled_launch<E, RL, NB, H, T, V, A, DIAG, true>(P, P.t_stage.as<V>(), x, s);
+      return;
+    }
+  }
+  auto kern = k_trsv_tiled<E, RL, NB, H, T, V, A, DIAG, STAGED>;
+  const size_t lds = tile_lds_bytes(P.t_ring, P.t_hmax, STAGED);
   static size_t lds_set = 0;  // per instantiation: the largest size allowed so far
   if (lds > lds_set) {
     LA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
@@ -1032,11 +1073,11 @@ void build_tiled(TrsvPlan &P, const std::vector<int> &iperm, const std::vector<i
   LA_HIP(hipGetDevice(&dev));
   LA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   LA_HIP(hipDeviceGetAttribute(&budget, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-  // halo slots: what LDS holds beyond the rings of kTileWindow groups (they
-  // are twice as long where the halo leaves room: the I/O wavefronts then
-  // run further ahead)
+  // halo slots: what LDS holds beyond the results of kTileWindow groups (and a
+  // ring of b as long, and both twice as long, where the halo leaves room: the
+  // I/O wavefronts then run further ahead)
   const int64_t avail =
-      static_cast<int64_t>(budget) - static_cast<int64_t>(tile_lds_bytes(kTileWindow, 0));
+      static_cast<int64_t>(budget) - static_cast<int64_t>(tile_lds_bytes(kTileWindow, 0, true));
   const int max_halo = static_cast<int>(avail / 8);
   if (max_halo < 128 || ncu < 1) {
     P.t_why = "LDS too small for the tiled schedule";
@@ -1052,11 +1093,12 @@ void build_tiled(TrsvPlan &P, const std::vector<int> &iperm, const std::vector<i
   const int64_t slots = static_cast<int64_t>(G + kTilePad) * kTileLanes, m = slots * E;
   std::vector<int> dpos(static_cast<size_t>(slots), -1);
   std::vector<int> lsrc(static_cast<size_t>(m), -1);
-  P.t_ring = tile_lds_bytes(2 * kTileWindow, L.h_max) <= static_cast<size_t>(budget)
+  P.t_ring = tile_lds_bytes(2 * kTileWindow, L.h_max, false) <= static_cast<size_t>(budget)
                  ? 2 * kTileWindow : kTileWindow;
+  const bool staged = tile_lds_bytes(P.t_ring, L.h_max, false) > static_cast<size_t>(budget);
   // byte addresses into LDS: the results of group i sit in place i % t_ring
-  const int zero = P.t_ring * kTileLanes;
-  std::vector<int> pcode(static_cast<size_t>(m), kTileCtl + 8 * zero), gtile(static_cast<size_t>(G));
+  const int zero = P.t_ring * kTileLanes, ctl = tile_ctl(staged);
+  std::vector<int> pcode(static_cast<size_t>(m), ctl + 8 * zero), gtile(static_cast<size_t>(G));
   for (int p = 0; p < L.nparts; ++p)
     for (int g = L.part_gptr[p]; g < L.part_gptr[p + 1]; ++g) gtile[g] = p;
   // a row of RL lanes: its first lane carries the row id, 1/d and the
@@ -1074,13 +1116,13 @@ void build_tiled(TrsvPlan &P, const std::vector<int> &iperm, const std::vector<i
           const size_t pe = static_cast<size_t>(sl) * E + e;
           const int c = L.tcode[te], q = L.tsrc[te];
           if (c < 0) {
-            pcode[pe] = kTileCtl + 8 * (zero + 1 + (-c - 1));
+            pcode[pe] = ctl + 8 * (zero + 1 + (-c - 1));
           } else if (q >= 0) {
             // the layout counts places modulo kTileWindow: the group is the
             // last one before this one at that place
             const int gi = g - L.part_gptr[gtile[g]];
             const int gd = gi - 1 - (gi - 1 - c / kTileLanes) % kTileWindow;
-            pcode[pe] = kTileCtl + 8 * (gd % P.t_ring * kTileLanes + c % kTileLanes);
+            pcode[pe] = ctl + 8 * (gd % P.t_ring * kTileLanes + c % kTileLanes);
           }
           lsrc[pe] = q >= 0 ? lrp[lpos[r]] + (q - P.h_ai[r]) : -1;
         }
@@ -1124,6 +1166,7 @@ void build_tiled(TrsvPlan &P, const std::vector<int> &iperm, const std::vector<i
                     zero + 1 + L.rf_slot[t]);
     }
   P.t_mail.alloc(sizeof(double) * static_cast<size_t>(P.t_nmail));
+  if (staged) P.t_stage.alloc(sizeof(double) * static_cast<size_t>(slots));
   auto up = [&](DevBuf &d, const void *h, size_t bytes) {
     d.alloc(std::max<size_t>(bytes, 4));
     d.upload(h, bytes, s);

@@ -580,3 +580,46 @@ def test_tiled_two_entries_a_row(dev, shape, val, vec):
         err = np.abs(x.cpu().numpy() - ref).max() / np.abs(ref).max()
         print("case", shape, val, vec, "upper" if upper else "lower", "err", err, flush=True)
         assert err <= (1e-12 if exact else 1e-4)
+
+
+@pytest.mark.parametrize("dims", [(2304, 6, 6), (2431, 6, 6), (8, 8, 4700), (8, 8, 4862)])
+@pytest.mark.parametrize("val", [la.F64, la.F32, la.BF16])
+def test_tiled_wide_halo(dev, dims, val):
+    """Tiles that read more than 18423 values of other tiles, up to the 19450
+    that fit beside the results: the right-hand side has no ring in LDS then.
+    Rows on four lanes (27-point ILU(1), 8 nx values) and on one (7-point, 4 nz
+    values). FP64 against the oracle, 1e-12. The others against the
+    level-by-level solve of the same plan: rows of at most 31 entries add at
+    most 32 roundings of 2^-24 on either side to what their inputs carry, and
+    the factors' off-diagonal row sums stay below 0.98, so 2 * 32 * 2^-24 /
+    0.02 = 1.9e-4 bounds the relative difference."""
+    import torch
+    F = la.iluk(la.gen.laplace3d(*dims), 0) if dims[0] == 8 else la.iluk(la.gen.aniso27(*dims), 1)
+    L, D, U = la.split_ldu(F)
+    b = la.gen.uniform(F.n, 29)
+    dt = torch.float64 if val == la.F64 else torch.float32
+    bt = torch.tensor(b, device=dev, dtype=dt)
+    for T, diag, upper in ((L, None, False), (U, D, True)):
+        S = la.TriangularSolve(T, diag, upper=upper)
+        assert S.info()["tiled"], dims
+        if val != la.F64:
+            S.add_dtype(val)
+        x, y = torch.zeros_like(bt), torch.zeros_like(bt)
+        S.solve(bt, x, val=val)
+        if val == la.F64:
+            o = orc.CSR(T.n, T.ai, T.aj, T.av)
+            ref = orc.backward_sub(o, D, b) if upper else orc.forward_sub(o, b)
+        else:
+            S.solve(bt, y, mode=la.TRSV_LEVEL, val=val)
+            ref = y.cpu().numpy()
+        err = np.abs(x.cpu().numpy() - ref).max() / np.abs(ref).max()
+        print("case", dims, val, "upper" if upper else "lower", "err", err, flush=True)
+        assert err <= (1e-12 if val == la.F64 else 2e-4)
+        S.solve(bt, y.zero_(), val=val)
+        assert torch.equal(x, y)
+
+
+def test_tiled_halo_limit(dev):
+    """One plane more than the LDS holds keeps the level-chunk schedule."""
+    L, D, U = la.split_ldu(la.iluk(la.gen.laplace3d(8, 8, 4863), 0))
+    assert not la.TriangularSolve(L, None, upper=False).info()["tiled"]
