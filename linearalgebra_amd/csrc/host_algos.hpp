@@ -86,6 +86,26 @@ bool build_tile_layout(int n, const int *ai, const int *aj, const int *level, in
                        int max_parts, int max_rows, int max_halo, TileLayout &out,
                        std::string &why);
 
+// Tiled solve (sptrsv.hip): groups whose rows sit in registers, which is one
+// block of its I/O wavefronts.
+constexpr int kTileDepth = 8;
+// The I/O wavefronts touch a block's records kTileAhead blocks ahead of the
+// solver, if the records between the two, over the tiles that are active at
+// a time (groups / levels), stay within kTileTouchBytes: with more, lines are
+// displaced before they are used and the touches only add traffic. Measured
+// per apply, with / without: 512^2 FP64 (1.8 MB) 372 / 386 us, 128^2 FP64
+// 171 / 182 us, 100x96x90 FP64 (6.5 MB) 200 / 210 us, 128^3 FP32 (7.0 MB)
+// 253 / 280 us, 128^3 FP64 (10.9 MB) 310 / 290 us, 90^3 27-point ILU(1) FP64
+// (11.3 MB) 1118 / 929 us; lower triangle of a 27-point operator on 1250 x 30
+// x 30 FP64 (8.9 MB, rings of 16 groups) 448 / 349 us. Three blocks ahead:
+// 2-4% slower than four.
+constexpr int kTileAhead = 4;
+constexpr int64_t kTileTouchBytes = 8 << 20;
+inline bool tile_touch(int64_t groups, int64_t levels, int64_t record_bytes) {
+  const int64_t active = groups / levels + 1;
+  return active * kTileAhead * kTileDepth * record_bytes <= kTileTouchBytes;
+}
+
 // Device factorisation (numeric.hip).
 // One sync-free launch, or one launch per level? The first gives every row as
 // many lanes as the longest one needs and keeps about 4096 wavefronts in

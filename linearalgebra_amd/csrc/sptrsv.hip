@@ -248,7 +248,6 @@ __global__ __launch_bounds__(NT) void k_trsv_syncfree(
 // what bounds the solve now. (With the hand-over slots alone the 3-D solves
 // gained 20-40%, but 512^2 lost 8%: one more store per group on the solver.)
 constexpr int kTileLanes = 64;
-constexpr int kTileDepth = 8;  // groups whose rows sit in registers; one block of the I/O wavefronts
 constexpr int kTileIo = 2;     // I/O wavefronts
 // bytes of LDS control words, ahead of the slots (a cache line, or what they
 // need where b is staged)
@@ -257,16 +256,6 @@ constexpr int tile_ctl(bool staged) { return staged ? 40 : 64; }
 // kTileDepth - 1 groups past a tile's last one and loads kTileDepth ahead),
 // and mail slots' spare groups per tile for the same reason.
 constexpr int kTilePad = 2 * kTileDepth;
-// The I/O wavefronts touch a block's records kTileAhead blocks ahead of the
-// solver, if the records between the two, over the tiles that are active at
-// a time (groups / levels), stay within kTileTouchBytes: with more, lines are
-// displaced before they are used and the touches only add traffic. Measured
-// per apply, with / without: 512^2 FP64 (1.8 MB) 372 / 386 us, 128^2 FP64
-// 171 / 182 us, 100x96x90 FP64 (6.5 MB) 200 / 210 us, 128^3 FP32 (7.0 MB)
-// 253 / 280 us, 128^3 FP64 (10.9 MB) 310 / 290 us, 90^3 27-point ILU(1) FP64
-// (11.3 MB) 1118 / 929 us. Three blocks ahead: 2-4% slower than four.
-constexpr int kTileAhead = 4;
-constexpr int64_t kTileTouchBytes = 8 << 20;
 constexpr int kTileNever = INT_MAX / 2;  // "all groups ready"
 
 __device__ __forceinline__ void lds_fence() {
@@ -827,8 +816,7 @@ void tiled_launch(TrsvPlan &P, const V *b, V *x, hipStream_t s) {
                                static_cast<int>(lds)));
     lds_set = lds;
   }
-  const int64_t active = P.t_ngroups / std::max(P.nlevels, 1) + 1;
-  const int touch = active * P.t_ring * TileRec<E, T>::kBytes <= kTileTouchBytes ? 1 : 0;
+  const int touch = tile_touch(P.t_ngroups, std::max(P.nlevels, 1), TileRec<E, T>::kBytes);
   const unsigned fg = static_cast<unsigned>(std::min<int64_t>(1024, (P.t_nmail + kB - 1) / kB));
   hipLaunchKernelGGL(k_tile_prep<V>, dim3(std::max(fg, 1u)), dim3(kB), 0, s, P.t_nmail,
                      P.t_mail.as<V>(), P.counter.as<unsigned>());

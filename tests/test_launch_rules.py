@@ -1,6 +1,6 @@
-"""Launch rules of the device factorisation (linearalgebra_amd/csrc/
-host_algos.hpp), called on the CPU (tests/cpp/factor_capi.cpp, built here
-with g++)."""
+"""Launch rules of the device factorisation and the tiled triangular solve
+(linearalgebra_amd/csrc/host_algos.hpp), called on the CPU (tests/cpp/
+launch_rules_capi.cpp, built here with g++)."""
 import ctypes as C
 import os
 import shutil
@@ -12,13 +12,13 @@ from helpers import ROOT
 
 
 @pytest.fixture(scope="module")
-def fac(tmp_path_factory):
+def rules(tmp_path_factory):
     if shutil.which("g++") is None:
         pytest.skip("needs g++")
-    so = str(tmp_path_factory.mktemp("factor") / "libfactor.so")
+    so = str(tmp_path_factory.mktemp("rules") / "librules.so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-shared", "-fPIC",
                     "-I", os.path.join(ROOT, "linearalgebra_amd", "csrc"), "-o", so,
-                    os.path.join(ROOT, "tests", "cpp", "factor_capi.cpp")],
+                    os.path.join(ROOT, "tests", "cpp", "launch_rules_capi.cpp")],
                    check=True, timeout=300)
     return C.CDLL(so)
 
@@ -27,10 +27,10 @@ def fac(tmp_path_factory):
     (1, 1, 1), (63, 1, 63), (1000, 1000, 64), (1000, 100, 120), (5000, 10, 1024),
     (178956970, 1, 1024), (178956971, 1, 1024), (2 ** 31 - 1, 1, 1024),
     (2 ** 31 - 1, 2 ** 28, 95), (2 ** 31 - 1, 2 ** 31 - 1, 64)])
-def test_workgroups(fac, chunks, levels, wgs):
+def test_factor_workgroups(rules, chunks, levels, wgs):
     """12 levels of chunks, at least 64 and at most 1024 workgroups, never
     more than there are chunks: up to the largest number of chunks."""
-    assert fac.fac_workgroups(chunks, levels) == wgs
+    assert rules.fac_workgroups(chunks, levels) == wgs
 
 
 @pytest.mark.parametrize("rows,levels,lanes,eliminations,one", [
@@ -48,7 +48,21 @@ def test_workgroups(fac, chunks, levels, wgs):
     (2000, 2, 64, 59, 1),
     (0, 1, 4, 0, 1),
     (2 ** 31 - 1, 3, 64, 2 ** 31 - 1, 0)])
-def test_one_launch(fac, rows, levels, lanes, eliminations, one):
+def test_factor_one_launch(rules, rows, levels, lanes, eliminations, one):
     """The faster form by measurement, on both sides of the line."""
-    assert fac.fac_one_launch(C.c_longlong(rows), C.c_longlong(levels), lanes,
+    assert rules.fac_one_launch(C.c_longlong(rows), C.c_longlong(levels), lanes,
                               C.c_longlong(eliminations)) == one
+
+
+@pytest.mark.parametrize("active,record,touch", [
+    (46, 5632, 1), (47, 5632, 0),      # eight FP64 values a lane: 8.29 / 8.47 MB
+    (78, 3328, 1), (79, 3328, 0),      # eight FP32 values
+    (73, 3584, 1), (74, 3584, 0),      # four FP64 values
+    (128, 2048, 1), (129, 2048, 0)])   # two FP64 values: 2^23 bytes exactly
+def test_tile_touch(rules, active, record, touch):
+    """Records between a touch and its use: four blocks of eight groups of
+    every active tile, however long the plan's rings are; 2^23 bytes at most."""
+    assert 32 * active * record <= 2 ** 23 if touch else 32 * active * record > 2 ** 23
+    levels = 1345
+    groups = C.c_longlong((active - 1) * levels + 7)
+    assert rules.tri_touch(groups, C.c_longlong(levels), C.c_longlong(record)) == touch
