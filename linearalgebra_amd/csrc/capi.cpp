@@ -31,6 +31,17 @@ void gen_diffusion2d(int nx, int ny, const double *theta, int *ai, int *aj, doub
 
 namespace {
 thread_local std::string tl_err;
+
+// the stream is being captured into a graph (or, the default stream, may not
+// be waited for because another one is)
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
 }
 void set_last_error(const std::string &m) { tl_err = m; }
 }  // namespace laamd
@@ -555,6 +566,10 @@ int la_prec_apply_transpose(la_prec_t P, la_trsv_mode mode, la_dtype val, la_dty
   LA_TRY
   LA_CHECK_ARG(P, "null handle");
   prec_apply_transpose(*P->p, mode, val, vec, r, z, P->p->stream);
+  // (a recorded apply has not run yet: the next checked call reports for it)
+  if (mode == LA_TRSV_SYNCFREE && !capturing(P->p->stream) &&
+      trsv_check_timeout({P->p->lower.get(), P->p->upper.get()}, P->p->stream))
+    throw la_error(LA_ERR_TIMEOUT, "sync-free triangular solve exceeded its spin bound");
   LA_CATCH
 }
 int la_prec_info(la_prec_t P, int *levels_lower, int *levels_upper) {
