@@ -288,3 +288,37 @@ def test_gram_schmidt_groups(dev, n, steps):
     assert full["converged"] and mixed["converged"]
     assert mixed["iters"] <= full["iters"] + k * mixed["outer_iters"]
     assert np.linalg.norm(r) <= 1.01e-9 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n", [3, 603, 524291])
+@pytest.mark.parametrize("steps", [1, 8, 9, 17, 25, 32, 33])
+def test_gram_schmidt_groups_fp32(dev, n, steps):
+    """One mixed-precision FGMRES cycle of a fixed number of steps, its
+    Gram-Schmidt kernels on FP32 vectors: fewer values than one load takes,
+    three left over, and more rows than one pass of the grid (2 x 131072 for
+    the two-value loads, 4 x 131072 for the four-value ones). The right-hand
+    side sits at the ends of the vectors and of those passes alone, and k
+    steps of the tridiagonal operator stay within k rows of it, so a value
+    left out there changes the iterate by parts of its norm. Against the FP64
+    iterate: basis, matrix and iterate are rounded to 2^-24, which the
+    operator (condition 51) carries on for k steps, 51 k 2^-24; 50 times that
+    is allowed."""
+    import torch
+    ai = np.concatenate([[0], np.cumsum(np.r_[2, np.full(n - 2, 3), 2])]).astype(np.int32)
+    aj = (np.repeat(np.arange(n), np.diff(ai)) +
+          np.concatenate([[0, 1], np.tile([-1, 0, 1], n - 2), [-1, 0]])).astype(np.int32)
+    av = np.choose(aj - np.repeat(np.arange(n), np.diff(ai)) + 1, [-0.9, 2.08, -1.1])
+    A = orc.CSR(n, ai, aj, av)
+    k = min(steps, n - 1)
+    b = np.zeros(n)
+    at = np.unique([t for e in (0, 262144, 524288, n) for t in range(e - 3, e + 3) if 0 <= t < n])
+    b[at] = la.gen.uniform(len(at), 9)
+    dA = la.DeviceMatrix(as_lib_csr(A))
+    x = torch.zeros(n, dtype=torch.float64, device=dev)
+    res = la.fgmres(dA, None, torch.tensor(b, device=dev), x, rel_tol=1e-30, restart=k,
+                    max_iters=k, inner_tol=1e-30, precision=la.PREC_MIXED_F32)
+    xo = orc.fgmres(A, b, restart=k, rel_tol=1e-30, maxiter=k)[0]
+    assert res["iters"] == k
+    err = np.linalg.norm(x.cpu().numpy() - xo) / np.linalg.norm(xo)
+    print("case", n, steps, "err", err, flush=True)
+    assert err <= 50 * 51 * k * 2.0 ** -24
