@@ -1178,6 +1178,11 @@ void build_tiled(TrsvPlan &P, const std::vector<int> &iperm, const std::vector<i
   tile_pack(P, LA_F64, s);
 }
 
+// LEVEL mode records at most this many levels in a graph. One of 131072 levels
+// ended in a segmentation fault of the host process (65536 ran), so longer
+// chains are launched level by level.
+constexpr int kGraphLevels = 65536;
+
 hipStream_t capture_stream() {
   static thread_local hipStream_t cs = nullptr;
   if (!cs) LA_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
@@ -1323,7 +1328,7 @@ void trsv_solve(TrsvPlan &T, la_trsv_mode mode, la_dtype val, la_dtype vec, cons
     return;
   }
   if ((T.nnz && !T.val.has[val]) || (!T.unit && !T.diag.has[val])) trsv_add_dtype(T, val);
-  if (mode == LA_TRSV_SYNCFREE || T.nlevels <= 2) {
+  if (mode == LA_TRSV_SYNCFREE || T.nlevels <= 2 || T.nlevels > kGraphLevels) {
     solve_dispatch(T, mode, val, vec, b, x, s);
     return;
   }
