@@ -235,9 +235,7 @@ bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes,
   part.assign(static_cast<size_t>(n), 0);
   tau = 0;
   nparts = 0;
-  auto tile_of = [&](int i, int t, int nv) {
-    return static_cast<size_t>(u[i] / t) * nv + v[i] / t;
-  };
+  std::vector<int> tile(static_cast<size_t>(n));  // at the edge tried
   // rows level by level and their groups in their tiles, when a larger edge
   // is tried
   std::vector<int> by_level, group;
@@ -245,7 +243,10 @@ bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes,
     const int nu = umax / t + 1, nv = vmax / t + 1;
     if (static_cast<int64_t>(nu) * nv > 4 * static_cast<int64_t>(max_parts)) continue;
     std::vector<int> cnt(static_cast<size_t>(nu) * nv, 0);
-    for (int i = 0; i < n; ++i) cnt[tile_of(i, t, nv)]++;
+    for (int i = 0; i < n; ++i) {
+      tile[i] = u[i] / t * nv + v[i] / t;
+      cnt[tile[i]]++;
+    }
     int used = 0, big = 0;
     for (int c : cnt) {
       used += c > 0;
@@ -277,7 +278,7 @@ bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes,
       bool fits = true;
       for (int k = 0; k < n && fits; ++k) {
         const int i = by_level[k];
-        const size_t c = tile_of(i, t, nv);
+        const int c = tile[i];
         if (seen[c] != level[i]) {
           seen[c] = level[i];
           rows[c] = 0;
@@ -286,7 +287,7 @@ bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes,
         group[i] = groups[c];
         fits = ++rows[c] <= lanes;
         for (int q = ai[i]; q < ai[i + 1]; ++q) {
-          const bool other = tile_of(aj[q], t, nv) != c;
+          const bool other = tile[aj[q]] != c;
           face[c] += other;
           cross += other;
           fits = fits && (other || group[i] - group[aj[q]] < kTileWindow);
@@ -299,7 +300,7 @@ bool bfs_tiles(int n, const int *ai, const int *aj, const int *level, int lanes,
     nparts = 0;
     for (size_t c = 0; c < cnt.size(); ++c)
       if (cnt[c]) id[c] = nparts++;
-    for (int i = 0; i < n; ++i) part[i] = id[tile_of(i, t, nv)];
+    for (int i = 0; i < n; ++i) part[i] = id[tile[i]];
     tau = t;
   }
   if (!tau) {
