@@ -308,7 +308,8 @@ int la_prec_set_stream(la_prec_t P, void *hip_stream);
 /* z = M^-1 r (device vectors). */
 int la_prec_apply(la_prec_t P, la_trsv_mode mode, la_dtype val, la_dtype vec,
                   const void *r, void *z);
-/* z = M^-T r. */
+/* z = M^-T r (sync-free: waits and reports LA_ERR_TIMEOUT like la_prec_apply,
+ * except while its stream is being captured). */
 int la_prec_apply_transpose(la_prec_t P, la_trsv_mode mode, la_dtype val,
                             la_dtype vec, const void *r, void *z);
 int la_prec_info(la_prec_t P, int *levels_lower, int *levels_upper);

@@ -92,13 +92,14 @@ constexpr int kTileDepth = 8;
 // The I/O wavefronts touch a block's records kTileAhead blocks ahead of the
 // solver, if the records between the two, over the tiles that are active at
 // a time (groups / levels), stay within kTileTouchBytes: with more, lines are
-// displaced before they are used and the touches only add traffic. Measured
-// per apply, with / without: 512^2 FP64 (1.8 MB) 372 / 386 us, 128^2 FP64
-// 171 / 182 us, 100x96x90 FP64 (6.5 MB) 200 / 210 us, 128^3 FP32 (7.0 MB)
-// 253 / 280 us, 128^3 FP64 (10.9 MB) 310 / 290 us, 90^3 27-point ILU(1) FP64
-// (11.3 MB) 1118 / 929 us; lower triangle of a 27-point operator on 1250 x 30
-// x 30 FP64 (8.9 MB, rings of 16 groups) 448 / 349 us. Three blocks ahead:
-// 2-4% slower than four.
+// displaced before they are used and the touches only add traffic. A lower
+// triangle with / without touches: 512^2 FP64 (0.5 MB) 158 / 169 us, 27-point
+// 24^3 FP64 (2.0 MB) 75 / 79 us, 7-point 128^3 FP32 (7.1 MB) 118 / 126 us,
+// 100^3 FP64 (7.4 MB) 99 / 106 us; 160^3 FP64 (16 MB) 493 / 422 us, 27-point
+// 112^3 FP32 (14 MB) 329 / 313 us, 96^3 FP64 (19 MB) 359 / 301 us. The line is
+// a compromise: 27-point FP64 already loses at 6-7 MB (56^3 186 / 178 us, 1250
+// x 22 x 22 394 / 320 us), 7-point 128^3 FP64 still gains at 11 MB (126 / 134
+// us). Three blocks ahead: 2-4% slower than four.
 constexpr int kTileAhead = 4;
 constexpr int64_t kTileTouchBytes = 8 << 20;
 inline bool tile_touch(int64_t groups, int64_t levels, int64_t record_bytes) {

@@ -241,8 +241,9 @@ __global__ __launch_bounds__(NT) void k_trsv_syncfree(
 // IC(0) FP64 425 -> 290 us, FP32 in natural order 631 -> 253 us; 100x96x90
 // FP64 494 -> 200 us; 512^2 FP64 569 -> 372 us; 128^2 225 -> 171 us; 27-point
 // ILU(1) 56^3 FP32 740 -> 447 us, 90^3 FP64 1470 -> 929 us (with larger tiles,
-// smaller records and one synchronisation per apply now 259, 222, 169, 303, 85,
-// 405 and 737 us in this order). A group takes the
+// smaller records and one synchronisation per apply now 259, 225, 172, 303, 85,
+// 407 and 736 us in this order, repeated on the same vectors; with others on
+// each pass 271 us for the first and 426 us for the sixth). A group takes the
 // solver 0.12 us (0.245 us before), and a hand-over about 1 us at the
 // median; the chain of hand-overs between tiles and of groups inside them is
 // what bounds the solve now. (With the hand-over slots alone the 3-D solves

@@ -623,3 +623,37 @@ def test_tiled_halo_limit(dev):
     """One plane more than the LDS holds keeps the level-chunk schedule."""
     L, D, U = la.split_ldu(la.iluk(la.gen.laplace3d(8, 8, 4863), 0))
     assert not la.TriangularSolve(L, None, upper=False).info()["tiled"]
+
+
+@pytest.mark.parametrize("order", ["back and forth", "two colours", "halves"])
+def test_tiled_row_orders(dev, order):
+    """Row orders whose tiles read each other or stay small for the LDS
+    window (128^2 5-point, rows back and forth; blocks of 32 x 32 nodes, one
+    colour first; two halves, then the column between them) are tiled and
+    solve to 1e-12 of the oracle, bitwise the same each time."""
+    import torch
+    m = 128
+    c = np.arange(m * m)
+    x, y = c % m, c // m
+    key = {"back and forth": y * m + np.where(y % 2 == 1, m - 1 - x, x),
+           "two colours": (x // 32 + y // 32) % 2 * m * m * m + (y // 32 * 4 + x // 32) * 1024 +
+                          y % 32 * 32 + x % 32,
+           "halves": np.where(x < m // 2, 0, np.where(x > m // 2, 1, 2)) * m * m + c}[order]
+    p = np.argsort(key, kind="stable").astype(np.int32)
+    ip = np.empty_like(p)
+    ip[p] = np.arange(m * m, dtype=np.int32)
+    A = la.permute(la.gen.poisson2d(m), p, ip)
+    L, D, U = la.split_ldu(la.iluk(A, 0))
+    b = la.gen.uniform(A.n, 37)
+    bt = torch.tensor(b, device=dev)
+    for T, diag, upper in ((L, None, False), (U, D, True)):
+        S = la.TriangularSolve(T, diag, upper=upper)
+        assert S.info()["tiled"], order
+        o = orc.CSR(T.n, T.ai, T.aj, T.av)
+        ref = orc.backward_sub(o, D, b) if upper else orc.forward_sub(o, b)
+        x1, x2 = torch.zeros_like(bt), torch.zeros_like(bt)
+        S.solve(bt, x1)
+        S.solve(bt, x2)
+        err = np.abs(x1.cpu().numpy() - ref).max() / np.abs(ref).max()
+        print("case", order, "upper" if upper else "lower", "err", err, flush=True)
+        assert err <= 1e-12 and torch.equal(x1, x2)
