@@ -124,11 +124,11 @@ inline bool factor_one_launch(int64_t rows, int64_t levels, int lanes, int64_t e
   const double per_level = 14000.0 * levels + 0.25 * rows + 0.28 * eliminations;
   return one <= per_level;
 }
-// Workgroups of the one launch: kFacAhead levels of chunks at a time (clamped to 64 .. 1024),
-// so that the pattern work of later rows is done while they wait. 27-point
-// ILU(1) on 48^3 with 1 / 2 / 4 / 8 / 16 levels ahead (8 wavefronts): 8.3 /
-// 6.1 / 3.4 / 2.3 / 2.2 ms; 72^3 IC(0) with 4 / 8 / 32: 490 / 465 / 573 us
-// (more pollers)
+// Workgroups of the one launch: kFacAhead levels of chunks at a time (clamped
+// to 64 .. 1024), so that the pattern work of later rows is done while they
+// wait. 27-point ILU(1) on 48^3 with 1 / 2 / 4 / 8 / 16 levels ahead (8
+// wavefronts): 8.3 / 6.1 / 3.4 / 2.3 / 2.2 ms; 72^3 IC(0) with 4 / 8 / 32: 490
+// / 465 / 573 us (more pollers)
 constexpr int64_t kFacAhead = 12;
 inline int factor_workgroups(int64_t chunks, int64_t levels) {
   return static_cast<int>(

@@ -250,8 +250,8 @@ __global__ __launch_bounds__(NT) void k_trsv_syncfree(
 // gained 20-40%, but 512^2 lost 8%: one more store per group on the solver.)
 constexpr int kTileLanes = 64;
 constexpr int kTileIo = 2;     // I/O wavefronts
-// bytes of LDS control words, ahead of the slots (a cache line, or what they
-// need where b is staged)
+// bytes of LDS control words, ahead of the slots (where b is staged no more
+// than they need: the halo is wide)
 constexpr int tile_ctl(bool staged) { return staged ? 40 : 64; }
 // Groups of padding the packed rows end with (the solver runs up to
 // kTileDepth - 1 groups past a tile's last one and loads kTileDepth ahead),
@@ -738,7 +738,8 @@ __global__ void k_tile_stage(int64_t slots, const int *__restrict__ dpos,
 // 8-byte LDS slots: results and, unless staged, b of `ring` groups, the zero
 // slot, the halo
 inline size_t tile_lds_bytes(int ring, int h_max, bool staged) {
-  return tile_ctl(staged) + 8 * ((staged ? 1 : 2) * static_cast<size_t>(ring) * kTileLanes + 1 + h_max);
+  const size_t rings = (staged ? 1 : 2) * static_cast<size_t>(ring) * kTileLanes;
+  return tile_ctl(staged) + 8 * (rings + 1 + h_max);
 }
 
 // The packed records: slot t's entries from the level-ordered values
